@@ -39,7 +39,10 @@ enum Counter : uint32_t {
   CNT_ERROR = 3,
   CNT_LIVE_NODES = 5,
   CNT_REACT_SATURATED = 6,  // particle-side reaction impulses clamped to the bins' range
-  CNT_COUNT = 8
+  CNT_COUNT = 8,
+  // in a cache line of its own: G2P counts here while every workgroup reads the line above
+  CNT_STRAYS = 32,          // entries of Topo::stray
+  CNT_WORDS = 64            // words of the counter array
 };
 // error bits in counters[CNT_ERROR]
 enum ErrorBit : uint32_t {
@@ -167,6 +170,23 @@ struct Parts {
   uint32_t stride;   // SoA capacity
 };
 
+// Which particles are in each particle block.  Block k's `meta` entry: x =
+// its first particles, idx[pblock_start[k] + k * pitch ...]; y = particles
+// that came from other blocks, the first kListRoom at idx[Topo::list_came +
+// k * kListRoom ...] and any beyond at idx[Topo::list_rest + z ...]; w = holes
+// (kInvalid) among the x.  After a full binning idx is the block-sorted list
+// and pitch 0; the lists that G2P writes for a listed substep (k_bin_update)
+// have room for pblock_len[k] + kListRoom first particles per block (pitch
+// kListRoom), and after a reorder are the block's storage range in order, with
+// a hole for each particle that left.
+constexpr uint32_t kListRoom = 64;
+struct BlockLists {
+  uint4* meta;
+  uint32_t* idx;
+  uint32_t pitch;
+  uint32_t pad;
+};
+
 struct Topo {
   uint32_t* owner;          // bucket -> owner id (0 empty, 1..n particle, > n neighbour insert)
   int4* bkey;               // bucket -> key, written by the claimer; x = kNoKey until then
@@ -178,6 +198,8 @@ struct Topo {
   int4* grid_key;           // slot -> (bx, by, bz, region)
   uint32_t grid_cap;
   uint32_t pblock_cap;
+  uint32_t grid_room;       // slots and particle blocks there is memory for: a listed substep keeps
+  uint32_t pblock_room;     // emptied blocks, beyond the capacities a full binning is held to
   uint32_t* pblock_nbr;     // 8 per particle block: buckets of block + {0,1}^3
   uint32_t* pblock_slot8;   // 8 grid slots per particle block
   uint32_t* pblock_start;
@@ -211,6 +233,17 @@ struct Topo {
   // mask of this substep; per bucket, the mask of its block key
   uint32_t* pmask;
   uint32_t* bmask;
+  // Listed substeps (k_bin_update): the block table of the last full binning
+  // stays, and each block's particles are those of its lists
+  uint32_t listed;          // this substep takes its particles from the lists `cur`
+  uint32_t build;           // this substep's G2P writes the next one's lists and keeps the block table
+  BlockLists cur;           // this substep's (the sorted list unless `listed`)
+  BlockLists nxt;           // written by G2P when `build` is set
+  uint64_t list_came, list_rest;  // parts of BlockLists::idx
+  // What k_bin_update has to place (counters[CNT_STRAYS] entries): a particle
+  // and the block whose entries for it are taken (its place beyond them is in
+  // pslot), or kInvalid where its block is to be looked up, and maybe made.
+  uint2* stray;
 };
 
 }  // namespace tmpm

@@ -17,6 +17,8 @@ void launch_cpic_mask(const Parts& p, const Topo& t, const DevClass* c, const De
                       hipStream_t s);
 void launch_bin_offsets(const Parts& p, const Topo& t, const DevClass* c, const DevScene* sc, hipStream_t s);
 void launch_bin_scatter(const Parts& p, const Topo& t, hipStream_t s);
+// in place of the four above in a listed substep (t.listed)
+void launch_bin_update(const Parts& p, const Topo& t, const DevClass* c, const DevScene* sc, hipStream_t s);
 void launch_p2g(const Parts& p, const Topo& t, const DevClass* c, const DevScene* sc, int fixed64, uint32_t blocks,
                 uint32_t threads, int copies, int plastic, hipStream_t s);
 // shapes != 0: some obstacle is a triangle prism or convex polyhedron

@@ -2,7 +2,9 @@
 //
 // Substep pipeline (all counts stay on the device; every kernel is a
 // grid-stride loop over a device-side count, so the launch sequence never
-// depends on host readback):
+// depends on host readback).  Kernels 1-4, a full binning, run in a substep
+// that reorders the particles; the substeps between two reorders keep the
+// block table and run k_bin_update in their place (see there):
 //   1 k_bin_insert        particle -> 4^3-cell block key, lock-free hash insert
 //                         by the head lane of each run of equal keys, counting-
 //                         sort rank; each workgroup lists the blocks it claimed
@@ -21,7 +23,8 @@
 //                         order, v = p/m + g dt, walls, obstacles
 //   7 k_g2p               per particle block: 6^3 velocity tile in LDS, gather,
 //                         v/C/x/F update, material projection, validity flags;
-//                         clears the block hash for the next substep
+//                         writes the next substep's block lists, or clears the
+//                         block hash before a full binning
 // The reference computes the same substep with an open-addressed hash of
 // all 27N stencil nodes (gpu_topology.wgsl:18-103) and per-particle CAS-loop
 // float atomics (gpu.wgsl:711-1019); here the hash holds blocks, not nodes,
@@ -48,6 +51,14 @@ __device__ __forceinline__ int readlane_i(int v, int lane) { return __builtin_am
 __device__ __forceinline__ int4 uniform4(int4 v) {
   return make_int4(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y),
                    __builtin_amdgcn_readfirstlane(v.z), __builtin_amdgcn_readfirstlane(v.w));
+}
+__device__ __forceinline__ uint32_t uniform1(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+// A value the compiler takes as a new one in each pass of a loop: what is
+// derived from it is computed there instead of being kept in registers over
+// the loop, which spilled them.
+__device__ __forceinline__ uint32_t per_pass(uint32_t v) {
+  asm volatile("" : "+v"(v));
+  return v;
 }
 __device__ __forceinline__ uint32_t readlane_u(uint32_t v, int lane) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
@@ -283,6 +294,44 @@ __device__ __forceinline__ void group_prefix(const uint32_t* const (&a)[K], uint
 __device__ __forceinline__ void clear_rev(const Topo& t, uint32_t slot) {
 #pragma unroll
   for (int d = 0; d < 8; ++d) t.grid_rev[8 * slot + d] = kInvalid;
+}
+
+// ---------------------------------------------------------------------------
+// Block lists of the listed substeps
+// ---------------------------------------------------------------------------
+// Particle i waits for k_bin_update: its block is to be looked up (kInvalid),
+// or block k has no entry left for it.
+__device__ __forceinline__ void stray_push(const Topo& t, uint32_t i, uint32_t k) {
+  t.stray[atomicAdd(&t.counters[CNT_STRAYS], 1u)] = make_uint2(i, k);
+}
+
+// Particle i comes into block k.
+__device__ __forceinline__ void list_came(const Topo& t, const BlockLists& l, uint32_t k, uint32_t i) {
+  const uint32_t pos = atomicAdd(&l.meta[k].y, 1u);
+  if (pos < kListRoom) {
+    l.idx[t.list_came + (uint64_t)kListRoom * k + pos] = i;
+  } else {
+    t.pslot[i] = pos - kListRoom;
+    stray_push(t, i, k);
+  }
+}
+
+// Where block k's particles are listed.  A particle's index is one load from a
+// selected address, so that several are in flight together.
+struct BlockParticles {
+  uint32_t total, stay, holes;
+  const uint32_t* stayed;  // the first `stay`
+  const uint32_t* came;    // the next kListRoom
+  const uint32_t* rest;    // those beyond
+};
+__device__ __forceinline__ BlockParticles block_particles(const Topo& t, uint32_t k, uint4 m, uint32_t start) {
+  return {m.x + m.y, m.x, m.w, t.cur.idx + start + (uint64_t)t.cur.pitch * k,
+          t.cur.idx + t.list_came + (uint64_t)kListRoom * k, t.cur.idx + t.list_rest + m.z};
+}
+// The j-th particle, j < total; kInvalid at a hole.
+__device__ __forceinline__ uint32_t block_particle(const BlockParticles& b, uint32_t j) {
+  const uint32_t a = j - b.stay;
+  return *(j < b.stay ? b.stayed + j : a < kListRoom ? b.came + a : b.rest + (a - kListRoom));
 }
 
 // ---------------------------------------------------------------------------
@@ -561,6 +610,7 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_offsets(Parts p, Topo t, co
       const uint32_t excl = wave_exclusive_scan(cnt, sum);
       if (mine) {
         t.pblock_start[pb] = carry + excl;
+        t.cur.meta[pb] = make_uint4(cnt, 0, 0, 0);
         t.bucket_start[b] = carry + excl;  // the scatter's one look-up per particle
       }
       carry += sum;
@@ -585,6 +635,7 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_offsets(Parts p, Topo t, co
     t.counters[CNT_PARTICLE_BLOCKS] = npb;
     t.counters[CNT_GRID_BLOCKS] = min(npb + total[1], t.grid_cap);
     t.counters[CNT_BINNED] = total[2];
+    t.counters[CNT_STRAYS] = 0;
   }
 }
 
@@ -632,6 +683,155 @@ __global__ __launch_bounds__(256) void k_bin_scatter(Parts p, Topo t) {
       else bad = true;  // offsets and ranks disagree: never write past the list
     }
     flag_error(t.counters, bad, ERR_INTERNAL);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Listed substeps: the blocks that particles entered without one
+// ---------------------------------------------------------------------------
+// A full binning (kernels 1-4) sorts every particle; between two reorders only
+// the few that change block need any of it.  G2P knows them: it writes each
+// block's list, its own particles that stay and those that come in from other
+// blocks, and what is left to do before the next P2G is to make the blocks
+// that particles entered and that do not exist yet.  Those particles
+// ("strays") are few, so one workgroup does it, its phases separated by barriers (which also order the
+// phases' memory accesses within the workgroup; device-wide fences between
+// them cost 2 us each): the strays' keys go
+// into the table, the first stray of each new particle block takes the next
+// id, the 7 upper neighbours of the new blocks go into the table, and the
+// tiles' slots and the lists are filled.  Blocks that particles have left stay
+// until the next full binning; their tiles are zero.  Every sum runs over the
+// same particles as after a full binning, in integers, so results are the same
+// bit for bit.
+//
+// In a kernel trace the four binning kernels took 39 us of a substep of 153 us
+// at 1M particles, 96 of 576 us at 4M and 19 of 52 us at 8k; this launch takes
+// 5 us without strays and 9 to 15 with some, and writing the lists 4 us of G2P at
+// 1M.
+constexpr int kUpdateThreads = 512;
+constexpr uint32_t kClaimed = kInvalid - 1;  // bucket_pblock of a block whose id is being taken
+
+__global__ __launch_bounds__(kUpdateThreads) void k_bin_update(Parts p, Topo t, const DevClass* classes,
+                                                               const DevScene* scenes) {
+  __shared__ uint32_t s_new, s_slots, s_rest;
+  const uint32_t strays = min(t.counters[CNT_STRAYS], p.n);
+  if (strays == 0) return;
+  const uint32_t tid = threadIdx.x;
+  const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS], ng = t.counters[CNT_GRID_BLOCKS],
+                 binned = t.counters[CNT_BINNED];
+  if (tid == 0) s_new = s_slots = s_rest = 0;
+  bool over = false;
+  // the buckets of the particles whose block is to be looked up (pslot: kInvalid for none)
+  for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
+    const uint2 e = t.stray[s];
+    if (e.y != kInvalid) continue;
+    const uint32_t i = e.x;
+    const DevClass& c = classes[p.cls[i]];
+    uint32_t b = kInvalid;
+    // as in k_bin_insert, a failed scene's particles are not binned any more
+    int3 cell;
+    if (!(t.isolate && t.scene_err[c.region >> 16] != 0u) && cell3(p.pos_mass[i], c.inv_h, cell)) {
+      bool claimed;
+      b = hash_insert<false, true>(p, t, classes, scenes,
+                                   make_int4(cell.x >> 2, cell.y >> 2, cell.z >> 2, (int)c.region), i + 1, claimed);
+      if (b == kInvalid) over = true;
+      else if (claimed) t.bucket_pblock[b] = t.bucket_slot[b] = kInvalid;
+    }
+    t.pslot[i] = b;
+  }
+  __syncthreads();
+  // grid slot of a bucket that has none
+  auto take_slot = [&](uint32_t b) {
+    const uint32_t slot = ng + atomicAdd(&s_slots, 1u);
+    if (slot >= t.grid_room) {
+      over = true;
+      return;
+    }
+    t.bucket_slot[b] = slot;
+    t.grid_key[slot] = t.bkey[b];
+    clear_rev(t, slot);
+  };
+  // new particle blocks: the first stray of each takes its id
+  for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
+    const uint2 e = t.stray[s];
+    const uint32_t b = e.y == kInvalid ? t.pslot[e.x] : kInvalid;
+    if (b == kInvalid || atomicCAS(&t.bucket_pblock[b], kInvalid, kClaimed) != kInvalid) continue;
+    const uint32_t pb = npb + atomicAdd(&s_new, 1u);
+    if (pb >= t.pblock_room) {
+      over = true;
+      continue;
+    }
+    if (t.bucket_slot[b] == kInvalid) take_slot(b);
+    t.pblock_nbr[8 * pb] = b;
+    t.pblock_start[pb] = binned;
+    t.pblock_len[pb] = 0;
+    t.cur.meta[pb] = make_uint4(0, 0, 0, 0);
+    t.bucket_pblock[b] = pb;
+  }
+  __syncthreads();
+  const uint32_t made = min(s_new, t.pblock_room - npb);
+  for (uint32_t q = tid; q < 7 * made; q += kUpdateThreads) {
+    const uint32_t pb = npb + q / 7u, d = q % 7u + 1u;
+    const uint32_t b = t.pblock_nbr[8 * pb];
+    int4 k = t.bkey[b];
+    k.x += (int)(d >> 2);
+    k.y += (int)((d >> 1) & 1);
+    k.z += (int)(d & 1);
+    bool claimed;
+    const uint32_t got = hash_insert<false, true>(p, t, classes, scenes, k, p.n + 1 + 8 * b + d, claimed);
+    if (got == kInvalid) {
+      over = true;
+    } else if (claimed) {
+      t.bucket_pblock[got] = t.bucket_slot[got] = kInvalid;
+      take_slot(got);
+    }
+    t.pblock_nbr[8 * pb + d] = got;
+  }
+  __syncthreads();
+  for (uint32_t q = tid; q < 8 * made; q += kUpdateThreads) {
+    const uint32_t pb = npb + (q >> 3), d = q & 7, b = t.pblock_nbr[8 * pb + d];
+    const uint32_t slot = b == kInvalid ? kInvalid : t.bucket_slot[b];
+    t.pblock_slot8[8 * pb + d] = slot;
+    if (slot != kInvalid) t.grid_rev[8 * slot + d] = pb;
+  }
+  // the strays' list entries; one beyond a block's entries becomes one with a block
+  for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
+    const uint2 e = t.stray[s];
+    const uint32_t i = e.x, b = e.y == kInvalid ? t.pslot[i] : kInvalid;
+    if (b == kInvalid) continue;
+    const uint32_t pb = t.bucket_pblock[b];
+    if (pb >= t.pblock_room) {  // no room for the block (flagged)
+      t.bucket_pblock[b] = kInvalid;
+      continue;
+    }
+    const uint32_t pos = atomicAdd(&t.cur.meta[pb].y, 1u);
+    if (pos < kListRoom) {
+      t.cur.idx[t.list_came + (uint64_t)kListRoom * pb + pos] = i;
+    } else {
+      t.pslot[i] = pos - kListRoom;
+      t.stray[s].y = pb;
+    }
+  }
+  __syncthreads();
+  // places for the particles beyond their blocks' entries: a run per block
+  for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
+    const uint2 e = t.stray[s];
+    if (e.y != kInvalid && t.pslot[e.x] == 0)
+      t.cur.meta[e.y].z = atomicAdd(&s_rest, atomicAdd(&t.cur.meta[e.y].y, 0u) - kListRoom);
+  }
+  __syncthreads();
+  for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
+    const uint2 e = t.stray[s];
+    if (e.y == kInvalid) continue;
+    const uint64_t at = (uint64_t)t.cur.meta[e.y].z + t.pslot[e.x];
+    if (at < p.n) t.cur.idx[t.list_rest + at] = e.x;
+    else atomicOr(&t.counters[CNT_ERROR], ERR_INTERNAL);  // more entries than particles: never write past them
+  }
+  flag_error(t.counters, over, ERR_TOPOLOGY);
+  if (tid == 0) {
+    t.counters[CNT_PARTICLE_BLOCKS] = npb + made;
+    t.counters[CNT_GRID_BLOCKS] = min(ng + s_slots, t.grid_room);
+    t.counters[CNT_STRAYS] = 0;
   }
 }
 
@@ -1622,17 +1822,23 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS
   static_assert(kTileNodes % 2 == 0 && kTile % 2 == 0, "tile planes hold whole node pairs");
   __shared__ uint32_t s_slot[8];
   const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS];
-  const int tid = threadIdx.x;
   for (uint32_t k = blockIdx.x; k < npb; k += gridDim.x) {
+    const int tid = (int)per_pass(threadIdx.x);
     // The block's particle range, slot list and the particle indices of the
     // first two passes load together, and the first particles' state loads
     // while the header (key, then scene) resolves: three dependent round trips
     // before any compute instead of five, and none for the second pass's
     // indices.
-    const uint32_t start = t.pblock_start[k], len = t.pblock_len[k];
+    const uint32_t start0 = t.pblock_start[k];
+    const uint4 meta0 = t.cur.meta[k];
     const uint32_t slot = tid < 8 ? t.pblock_slot8[8 * k + tid] : 0u;
-    const uint32_t i_first = (uint32_t)tid < len ? t.sorted[start + tid] : 0u;
-    const uint32_t i_second = (uint32_t)(tid + THREADS) < len ? t.sorted[start + tid + THREADS] : 0u;
+    const uint32_t start = uniform1(start0);
+    const BlockParticles list = block_particles(
+        t, k, make_uint4(uniform1(meta0.x), uniform1(meta0.y), uniform1(meta0.z), uniform1(meta0.w)), start);
+    const uint32_t total = list.total;
+    const uint32_t i_first = (uint32_t)tid < total ? block_particle(list, tid) : 0u;
+    const uint32_t i_second = (uint32_t)(tid + THREADS) < total ? block_particle(list, tid + THREADS) : 0u;
+    if (t.build && tid == 0) t.nxt.meta[k] = make_uint4(0, 0, 0, 0);  // this substep's G2P fills the lists
     if (tid < 8) s_slot[tid] = slot;
     for (int q = tid; q < COPIES * kTile / 2; q += THREADS) reinterpret_cast<ulonglong2*>(tacc)[q] = make_ulonglong2(0, 0);
     __syncthreads();
@@ -1649,9 +1855,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS
     const float stress_scale = -sc.dt * sc.inv_d;
     const float mscale = exp2f((float)sc.mass_shift), pscale = exp2f((float)sc.mom_shift);
     const int ox = key.x * kBlockCells, oy = key.y * kBlockCells, oz = key.z * kBlockCells;
-    bool bad = false, range = len > kP2GMaxBlock;
-    for (uint32_t j = tid; j < len; j += THREADS) {
-      const uint32_t i = j == (uint32_t)tid ? i_first : j == (uint32_t)(tid + THREADS) ? i_second : t.sorted[start + j];
+    bool bad = false, range = total - list.holes > kP2GMaxBlock;
+    for (uint32_t j = tid; j < total; j += THREADS) {
+      const uint32_t i = j == (uint32_t)tid               ? i_first
+                         : j == (uint32_t)(tid + THREADS) ? i_second
+                                                          : block_particle(list, j);
+      if (i == kInvalid) continue;  // a hole
       const float4 pm = p.pos_mass[i];
       const float4 vv = p.vel_vol[i];
       const DevClass& cls = classes[p.cls[i]];
@@ -1909,6 +2118,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && 
   __shared__ unsigned long long s_level_cells[MOVE ? kMoveLevels : 1];
   __shared__ uint32_t s_level_start[MOVE ? kMoveLevels : 1];
   __shared__ uint32_t s_levels;
+  // the next substep's lists: particles that stay in the block, and those that leave it
+  __shared__ uint32_t s_stay, s_left;
+  __shared__ uint32_t s_nbr[16];  // particle blocks at key + d (d = 0..7), then at key - d
   // Particle-side reactions (REACT) on a scene's first kMaxReactObstacles
   // obstacles: each contact adds its rounded impulse (reaction_fixed) into
   // these workgroup sums, which go to the obstacle's bins once per block.
@@ -1924,9 +2136,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && 
       q.ins_id[i] = kInvalid;
     }
   }
-  // The block hash is not read after the scatter of this substep: clear it
-  // here for the next substep's binning (saves a launch).
-  {
+  // Before a full binning the block hash, which is not read any more in this
+  // substep, is cleared here (saves a launch); a listed substep keeps it.
+  if (!t.build) {
     const uint32_t nb = t.bucket_mask + 1;
     for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < nb; b += gridDim.x * blockDim.x) {
       t.owner[b] = 0;
@@ -1938,22 +2150,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && 
   for (uint32_t v = blockIdx.x; v < span; v += gridDim.x) {
     const uint32_t k = xcd_block(v, npb, gridDim.x);
     if (k >= npb) continue;  // uniform over the workgroup
+    const uint32_t tid = per_pass(threadIdx.x);
     // As in P2G: the block's particle range, slot list and the particle
     // indices of the first two passes load together, and the block key loads
     // with the velocity tile.
-    const uint32_t start = t.pblock_start[k], len = t.pblock_len[k];
-    const uint32_t slot0 = threadIdx.x < 8 ? t.pblock_slot8[8 * k + threadIdx.x] : 0u;
-    const uint32_t i_first = threadIdx.x < len ? t.sorted[start + threadIdx.x] : 0u;
-    const uint32_t i_second = threadIdx.x + blockDim.x < len ? t.sorted[start + threadIdx.x + blockDim.x] : 0u;
-    if (threadIdx.x < 8) s_slot[threadIdx.x] = slot0;
+    const uint32_t start0 = t.pblock_start[k], len0 = t.pblock_len[k];
+    const uint4 meta0 = t.cur.meta[k];
+    const uint32_t slot0 = tid < 8 ? t.pblock_slot8[8 * k + tid] : 0u;
+    const uint32_t start = uniform1(start0), len = uniform1(len0);
+    const BlockParticles list = block_particles(
+        t, k, make_uint4(uniform1(meta0.x), uniform1(meta0.y), uniform1(meta0.z), uniform1(meta0.w)), start);
+    const uint32_t total = list.total;
+    const uint32_t i_first = tid < total ? block_particle(list, tid) : 0u;
+    const uint32_t i_second = tid + blockDim.x < total ? block_particle(list, tid + blockDim.x) : 0u;
+    if (tid == 0) s_stay = s_left = 0;
+    if (tid < 8) s_slot[tid] = slot0;
     if (REACT)  // the previous block's sums were flushed before the loop's last barrier
-      for (int q = threadIdx.x; q < kReactSums; q += blockDim.x) rsum[q] = 0ull;
+      for (int q = tid; q < kReactSums; q += blockDim.x) rsum[q] = 0ull;
     __syncthreads();
     // uniform over the workgroup: the block key, the scene and its obstacles
     // then load as scalars
     const uint32_t own = __builtin_amdgcn_readfirstlane(s_slot[0]);
     const int4 key = own != kInvalid ? uniform4(t.grid_key[own]) : make_int4(0, 0, 0, 0);
-    for (int n = threadIdx.x; n < kTileNodes; n += blockDim.x) {
+    // grid block s's own particle block is grid_rev[8 s], the one d below it grid_rev[8 s + d]
+    uint32_t nbr = kInvalid;
+    if (t.build && tid < 16 && own != kInvalid) {
+      const uint32_t d = tid & 7, s = tid < 8 ? s_slot[d] : own;
+      if (s != kInvalid) nbr = t.grid_rev[8 * s + (tid < 8 ? 0u : d)];
+    }
+    for (int n = tid; n < kTileNodes; n += blockDim.x) {
       int d, local;
       tile_node(n, d, local);
       uint32_t slot = s_slot[d];
@@ -1963,18 +2188,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && 
       vt[kTileNodes + n] = v.y;
       vt[2 * kTileNodes + n] = v.z;
     }
+    if (tid < 16) s_nbr[tid] = nbr;
     __syncthreads();
     if (own != kInvalid) {
       const DevScene& sc = scenes[(uint32_t)key.w >> 16];
       const float h = sc.h, inv_h = sc.inv_h, dt = sc.dt, inv_d = sc.inv_d;
       const int ox = key.x * kBlockCells, oy = key.y * kBlockCells, oz = key.z * kBlockCells;
       bool failed = false, bad = false;
+      // Particle w stays in the block: the next entry of its list, in the
+      // order of the passes.  False when the block has no entry left.
+      auto list_stay = [&](uint32_t w) {
+        if (MOVE) {  // the entry of its slot: the list keeps the reorder's order
+          t.nxt.idx[w + (uint64_t)kListRoom * k] = w;
+          return true;
+        }
+        const uint64_t m = __ballot(true);
+        const uint32_t lead = (uint32_t)__ffsll((unsigned long long)m) - 1;
+        uint32_t at = 0;
+        if (lane_id() == lead) at = atomicAdd(&s_stay, (uint32_t)__popcll(m));
+        at = readlane_u(at, lead) + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        if (at >= len + kListRoom) return false;
+        t.nxt.idx[start + (uint64_t)kListRoom * k + at] = w;
+        return true;
+      };
+      // Particle w goes on another list.  Nearly all that leave enter a block
+      // a step up or a step down along each axis, known from the grid blocks
+      // at hand; the others are looked up by k_bin_update.
+      auto list_later = [&](uint32_t w, int dx, int dy, int dz) {
+        if (MOVE) t.nxt.idx[w + (uint64_t)kListRoom * k] = kInvalid;
+        const bool up = ((dx | dy | dz) & ~1) == 0, down = ((-dx | -dy | -dz) & ~1) == 0;
+        const uint32_t into = up ? s_nbr[4 * dx + 2 * dy + dz] : down ? s_nbr[8 - 4 * dx - 2 * dy - dz] : kInvalid;
+        if (MOVE) atomicAdd(&s_left, 1u);
+        if (into != kInvalid) list_came(t, t.nxt, into, w);
+        else stray_push(t, w, kInvalid);
+      };
       const bool spread = move && len <= kMoveOrderMax;  // uniform over the workgroup
       if (spread) {
-        for (uint32_t c = threadIdx.x; c < 65; c += blockDim.x) s_cnt[c] = 0;
+        for (uint32_t c = tid; c < 65; c += blockDim.x) s_cnt[c] = 0;
         __syncthreads();
-        for (uint32_t j = threadIdx.x; j < len; j += blockDim.x) {
-          const uint32_t i = j == threadIdx.x ? i_first : j == threadIdx.x + blockDim.x ? i_second : t.sorted[start + j];
+        for (uint32_t j = tid; j < len; j += blockDim.x) {
+          const uint32_t i = j == tid ? i_first : j == tid + blockDim.x ? i_second : t.sorted[start + j];
           int3 cell;
           cell3(p.pos_mass[i], inv_h, cell);
           const int lx = cell.x - ox, ly = cell.y - oy, lz = cell.z - oz;
@@ -1988,32 +2241,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && 
         // of every cell with more than r particles, in cell order (cell 64,
         // the particles outside the block, last).  The first wavefront, one
         // lane per cell, lists each level's cells and where the level starts.
-        if (threadIdx.x < 64) {
-          const uint32_t n = s_cnt[threadIdx.x], outside = s_cnt[64];
+        if (tid < 64) {
+          const uint32_t n = s_cnt[tid], outside = s_cnt[64];
           uint32_t level = 0, at = 0;
           for (; level < kMoveLevels; ++level) {
             const uint64_t cells = __ballot(n > level);
             if (cells == 0 && outside <= level) break;  // uniform over the wavefront
-            if (threadIdx.x == 0) {
+            if (tid == 0) {
               s_level_cells[level] = cells;
               s_level_start[level] = at;
             }
             at += (uint32_t)__popcll(cells) + (outside > level ? 1u : 0u);
           }
           const uint64_t beyond = __ballot(n > level);  // after a full loop: cells past the last level
-          if (threadIdx.x == 0) s_levels = level < kMoveLevels || (beyond == 0 && outside <= level) ? level : kMoveLevels + 1;
+          if (tid == 0) s_levels = level < kMoveLevels || (beyond == 0 && outside <= level) ? level : kMoveLevels + 1;
         }
         __syncthreads();
         const bool by_level = s_levels <= kMoveLevels;  // else a cell holds too many particles
-        for (uint32_t j = threadIdx.x; j < len; j += blockDim.x) {
+        for (uint32_t j = tid; j < len; j += blockDim.x) {
           const uint32_t lc = s_dest[j] >> 16, r = min(s_dest[j] & 0xffffu, kMoveLevels - 1);
           const unsigned long long lower = lc < 64 ? (1ull << lc) - 1ull : ~0ull;
           // entry j is only read by this thread
           s_dest[j] = by_level ? s_level_start[r] + (uint32_t)__popcll(s_level_cells[r] & lower) : j;
         }
       }
-      for (uint32_t j = threadIdx.x; j < len; j += blockDim.x) {
-        const uint32_t i = j == threadIdx.x ? i_first : j == threadIdx.x + blockDim.x ? i_second : t.sorted[start + j];
+      for (uint32_t j = tid; j < total; j += blockDim.x) {
+        const uint32_t i = j == tid                ? i_first
+                           : j == tid + blockDim.x ? i_second
+                                                           : block_particle(list, j);
+        if (i == kInvalid) continue;  // a hole
         // the slot the particle is written to
         const uint32_t w = move ? start + (spread ? s_dest[j] : j) : i;
         const float4 pm = p.pos_mass[i];
@@ -2029,6 +2285,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && 
           }
         };
         if (cl.fixed) {
+          if (t.build && !list_stay(w)) list_later(w, 0, 0, 0);
           const float4 vv = p.vel_vol[i];
           o.vel_vol[w] = make_float4(0.f, 0.f, 0.f, vv.w);
           if (sc.apply_force) p.force[p.ins_id[i]] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -2140,6 +2397,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && 
             }
           }
         }
+        // The new cell: still in the grid?  Then the next substep's lists (a
+        // particle that left the representable cells is on none).  Here rather
+        // than after the state is written, where the cell would be live over
+        // the deformation update and spill.
+        {
+          int3 nb;
+          const bool ok = cell3(make_float4(x.x, x.y, x.z, 0.f), inv_h, nb);
+          failed |= !ok || nb.x < sc.first_base[0] || nb.y < sc.first_base[1] || nb.z < sc.first_base[2] ||
+                    nb.x > sc.last_base[0] || nb.y > sc.last_base[1] || nb.z > sc.last_base[2];
+          if (MOVE && t.build && !ok) {
+            t.nxt.idx[w + (uint64_t)kListRoom * k] = kInvalid;
+          } else if (t.build && ok) {
+            const int dx = (nb.x >> 2) - key.x, dy = (nb.y >> 2) - key.y, dz = (nb.z >> 2) - key.z;
+            if ((dx | dy | dz) != 0 || !list_stay(w)) list_later(w, dx, dy, dz);
+          }
+        }
         // F <- (I + C dt) F
         M3 Fo, Fn;
 #pragma unroll
@@ -2170,23 +2443,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && 
         }
         if (move) carry(!plastic_written);
         // Resident validity (gpu.wgsl:946-993).
-        int3 nb;
-        bool ok = cell3(make_float4(x.x, x.y, x.z, 0.f), inv_h, nb);
         bool fin = finite_abs(x.x) && finite_abs(x.y) && finite_abs(x.z) && finite_abs(v.x) && finite_abs(v.y) &&
                    finite_abs(v.z);
 #pragma unroll
         for (int q = 0; q < 9; ++q) fin = fin && finite_abs(Fn.a[q]);
         fin = fin && finite_abs(c0.x) && finite_abs(c0.y) && finite_abs(c0.z) && finite_abs(c1.x) &&
               finite_abs(c1.y) && finite_abs(c1.z) && finite_abs(c2.x) && finite_abs(c2.y) && finite_abs(c2.z);
-        bool out = !ok || nb.x < sc.first_base[0] || nb.y < sc.first_base[1] || nb.z < sc.first_base[2] ||
-                   nb.x > sc.last_base[0] || nb.y > sc.last_base[1] || nb.z > sc.last_base[2];
         const float density = fmaxf(pm.w / p.vel_vol[i].w, 1e-12f);
         const float wave = sqrtf(cl.wave_numerator / density);
         // sand-NH: wave speed at the current volume, 0.5 h bound (material.rs:388-396)
         const bool cfl = PLASTIC && cl.kind == DM_SAND_NH
                              ? dt * fmaxf(wave * sqrtf(fmaxf(det3(Fn), 1e-6f)), len3(v)) > 0.5f * h * (1.0f + 1e-4f)
                              : dt * (wave + len3(v)) > 0.4f * h * (1.0f + 1e-4f);
-        failed |= out || !fin || cfl;
+        failed |= !fin || cfl;
         o.pos_mass[w] = make_float4(x.x, x.y, x.z, pm.w);
         const float vol = p.vel_vol[i].w;
         o.vel_vol[w] = make_float4(v.x, v.y, v.z, vol);
@@ -2196,13 +2465,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && 
 #pragma unroll
         for (int a = 0; a < 9; ++a) o.F[a * o.stride + w] = Fn.a[a];
       }
+      if (t.build) {  // uniform over the workgroup, as own is
+        __syncthreads();
+        if (tid == 0) {
+          t.nxt.meta[k].x = MOVE ? len : min(s_stay, len + kListRoom);
+          if (MOVE) t.nxt.meta[k].w = s_left;
+        }
+      }
       flag_scene_error(t, (uint32_t)key.w >> 16, failed, ERR_RESIDENT);
       flag_error(t.counters, bad, ERR_INTERNAL);
       if (REACT) {  // own is uniform over the workgroup: every thread reaches the barrier
         __syncthreads();
         const int sums = min(sc.obstacle_count, kMaxReactObstacles) * 6;
         unsigned long long* bins = reinterpret_cast<unsigned long long*>(t.react_bins);
-        for (int q = threadIdx.x; q < sums; q += blockDim.x) {
+        for (int q = tid; q < sums; q += blockDim.x) {
           const unsigned long long v = rsum[q];
           if (v) atomicAdd(&bins[((size_t)(sc.obstacle_begin + q / 6) * kReactBins + k % kReactBins) * 6 + q % 6], v);
         }
@@ -2654,6 +2930,9 @@ void launch_bin_offsets(const Parts& p, const Topo& t, const DevClass* c, const 
 }
 void launch_bin_scatter(const Parts& p, const Topo& t, hipStream_t s) {
   hipLaunchKernelGGL(k_bin_scatter, dim3(grid_for(p.n, 256 * kScatterK, 2048)), dim3(256), 0, s, p, t);
+}
+void launch_bin_update(const Parts& p, const Topo& t, const DevClass* c, const DevScene* sc, hipStream_t s) {
+  hipLaunchKernelGGL(k_bin_update, dim3(1), dim3(kUpdateThreads), 0, s, p, t, c, sc);
 }
 void launch_p2g(const Parts& p, const Topo& t, const DevClass* c, const DevScene* sc, int fixed64, uint32_t blocks,
                 uint32_t threads, int copies, int plastic, hipStream_t s) {

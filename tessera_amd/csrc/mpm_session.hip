@@ -656,7 +656,10 @@ struct tmpm_session {
   // topology
   DevBuf owner, bkey, bucket_count, bucket_start, bucket_slot, bucket_pblock, grid_key, pblock_nbr,
       pblock_slot8, pblock_start, pblock_len, pslot, prank, sorted, counters, ptile, grid_rev, grid_vel, node_mask,
-    bin_stage, bin_nstage, bin_claims, bin_nclaims, bin_csum, bmask, pmask;
+    bin_stage, bin_nstage, bin_claims, bin_nclaims, bin_csum, bmask, pmask, stray;
+  DevBuf list_meta[2], list_idx[2];  // block lists, read and written in turn
+  bool lists_valid = false;  // the last substep left the next one's block lists and the block table
+  int list_read = 0;         // the set the next listed substep reads
   Topo topo{};
   uint32_t p2g_blocks = 4096, threads_pblock = 64, p2g_threads = 64;
   bool p2g_shape_fixed = false;  // P2G shape set by the tuner or an override, not by scene size
@@ -704,7 +707,8 @@ struct tmpm_session {
           &react_bins, &react_sub, &react_total, &rigid, &rigid_maps, &body_scene, &owner, &bkey, &bucket_count,
           &bucket_start, &bucket_slot, &bucket_pblock, &grid_key, &pblock_nbr, &pblock_slot8, &pblock_start,
           &pblock_len, &pslot, &prank, &sorted, &counters, &ptile, &grid_rev, &grid_vel, &node_mask, &bin_stage,
-          &bin_nstage, &bin_claims, &bin_nclaims, &bin_csum, &bmask, &pmask, &audit_dev})
+          &bin_nstage, &bin_claims, &bin_nclaims, &bin_csum, &bmask, &pmask, &stray, &list_meta[0], &list_meta[1],
+          &list_idx[0], &list_idx[1], &audit_dev})
       add(*d);
     return total;
   }
@@ -1099,10 +1103,21 @@ void read_tuning_env(tmpm_session* s) {
   }
 }
 
+BlockLists block_lists(const tmpm_session* s, int set) {
+  return {s->list_meta[set].as<uint4>(), s->list_idx[set].as<uint32_t>(), kListRoom, 0};
+}
+
 // Allocates the topology for `pblocks` particle blocks and `gblocks` grid
 // blocks of capacity.
 tmpm_status alloc_topology(tmpm_session* s, uint32_t pblock_cap, uint32_t grid_cap) {
   pblock_cap = std::min(pblock_cap, grid_cap);  // a particle block's grid slot is its id
+  // Listed substeps keep the blocks that particles have left until the next
+  // full binning: memory beyond the capacities, so that those cannot make a
+  // scene fail that a full binning of every substep would fit.
+  const uint32_t ncap = std::max<uint32_t>(s->cap, 1);
+  const uint32_t grid_room = grid_cap + grid_cap / 2;
+  const uint32_t pblock_room =
+      (uint32_t)std::max<uint64_t>(2ull * pblock_cap, std::min<uint64_t>(8ull * ncap, (uint64_t)kMinBuckets));
   uint32_t buckets = std::max<uint32_t>(next_pow2(2ull * grid_cap), (uint32_t)kMinBuckets);
   if ((uint64_t)s->cap + 8ull * buckets + 1 >= 0xffffffffull) return fail(TMPM_CAPACITY, "topology id space exhausted");
   Topo& t = s->topo;
@@ -1113,18 +1128,30 @@ tmpm_status alloc_topology(tmpm_session* s, uint32_t pblock_cap, uint32_t grid_c
   HIP_TRY(s->bucket_start.alloc(4ull * buckets));
   HIP_TRY(s->bucket_slot.alloc(4ull * buckets));
   HIP_TRY(s->bucket_pblock.alloc(4ull * buckets));
-  HIP_TRY(s->grid_key.alloc(16ull * grid_cap));
-  HIP_TRY(s->pblock_nbr.alloc(32ull * pblock_cap));
-  HIP_TRY(s->pblock_slot8.alloc(32ull * pblock_cap));
-  HIP_TRY(s->pblock_start.alloc(4ull * pblock_cap));
-  HIP_TRY(s->pblock_len.alloc(4ull * pblock_cap));
+  HIP_TRY(s->grid_key.alloc(16ull * grid_room));
+  HIP_TRY(s->pblock_nbr.alloc(32ull * pblock_room));
+  HIP_TRY(s->pblock_slot8.alloc(32ull * pblock_room));
+  HIP_TRY(s->pblock_start.alloc(4ull * pblock_room));
+  HIP_TRY(s->pblock_len.alloc(4ull * pblock_room));
+  for (int l = 0; l < 2; ++l) {
+    HIP_TRY(s->list_meta[l].alloc(16ull * pblock_room));
+    HIP_TRY(s->list_idx[l].alloc(4ull * (2ull * ncap + 2ull * kListRoom * pblock_room)));
+  }
+  HIP_TRY(s->stray.alloc(8ull * ncap));
+  t.cur.meta = s->list_meta[0].as<uint4>();  // what a full binning writes
+  t.list_rest = (uint64_t)ncap + 2ull * kListRoom * pblock_room;
+  t.list_came = (uint64_t)ncap + (uint64_t)kListRoom * pblock_room;
+  t.stray = s->stray.as<uint2>();
+  t.grid_room = grid_room;
+  t.pblock_room = pblock_room;
+  s->lists_valid = false;
   s->topo_cap = s->cap;
   HIP_TRY(s->pslot.alloc(4ull * std::max<uint32_t>(s->cap, 1)));
   HIP_TRY(s->prank.alloc(4ull * std::max<uint32_t>(s->cap, 1)));
   HIP_TRY(s->sorted.alloc(4ull * std::max<uint32_t>(s->cap, 1)));
   HIP_TRY(s->pmask.alloc(4ull * std::max<uint32_t>(s->cap, 1)));
-  HIP_TRY(s->counters.alloc(4ull * CNT_COUNT));
-  HIP_TRY(hipMemset(s->counters.ptr, 0, 4ull * CNT_COUNT));
+  HIP_TRY(s->counters.alloc(4ull * CNT_WORDS));
+  HIP_TRY(hipMemset(s->counters.ptr, 0, 4ull * CNT_WORDS));
   // Binning workgroups: at most ~2048 (each one's id prefix sums over all of
   // them), each over a whole number of 256-particle rounds.
   const uint64_t nparts = std::max<uint32_t>(s->cap, 1);
@@ -1142,10 +1169,10 @@ tmpm_status alloc_topology(tmpm_session* s, uint32_t pblock_cap, uint32_t grid_c
   t.bin_claims = s->bin_claims.as<uint32_t>();
   t.bin_nclaims = s->bin_nclaims.as<uint32_t>();
   t.bin_csum = s->bin_csum.as<uint32_t>();
-  HIP_TRY(s->ptile.alloc((size_t)grid_cap * kTileNodes * (s->fixed64 ? 32 : 16)));
-  HIP_TRY(s->grid_rev.alloc(32ull * grid_cap));
-  HIP_TRY(s->grid_vel.alloc((size_t)grid_cap * kBlockNodes * 16));
-  HIP_TRY(s->node_mask.alloc(8ull * grid_cap));
+  HIP_TRY(s->ptile.alloc((size_t)grid_room * kTileNodes * (s->fixed64 ? 32 : 16)));
+  HIP_TRY(s->grid_rev.alloc(32ull * grid_room));
+  HIP_TRY(s->grid_vel.alloc((size_t)grid_room * kBlockNodes * 16));
+  HIP_TRY(s->node_mask.alloc(8ull * grid_room));
   t.owner = s->owner.as<uint32_t>();
   t.bkey = s->bkey.as<int4>();
   t.bmask = s->bmask.as<uint32_t>();
@@ -1653,6 +1680,7 @@ tmpm_status prepare(tmpm_session* s) {
 tmpm_status prepare_packed(tmpm_session* s, PackedParticles& pk) {
   s->prepared = false;
   s->topo_valid = false;
+  s->lists_valid = false;
   if (s->scenes.size() > 0xffffu) return fail(TMPM_CAPACITY, "too many scenes");
   uint64_t total = 0;
   for (auto& scene : s->scenes) {
@@ -1735,6 +1763,7 @@ hipError_t enqueue_binning(tmpm_session* s, const Parts& p) {
   const DevScene* sc = s->scene_plain.as<DevScene>();
   Topo& t = s->topo;
   hipError_t e;
+  s->lists_valid = false;  // the table and the blocks' ranges are made anew
   if (s->table_dirty) {
     if ((e = timed(s, "k_topo_clear", [&] { launch_topo_clear(t, s->stream); })) != hipSuccess) return e;
     s->table_dirty = false;
@@ -1918,13 +1947,36 @@ void effective_p2g_shape(const tmpm_session* s, uint32_t& threads, int& copies) 
   copies = 1;
 }
 
+// Listed substeps.  A substep after a reorder takes its particles from the
+// blocks' ranges and lists (k_bin_update) for as long as the lists are whole:
+// no edit of the particles, no topology change and at most kListSpan substeps
+// since the reorder, so that lists stay short.  With CPIC a particle changes
+// its block key without moving to another cell: every substep bins fully.
+// Where lists are lost, the next substep bins fully and reorders, unless the
+// reorder interval is beyond the span (then only its own reorders happen).
+constexpr uint32_t kListSpan = 32;
+
 SubstepPlan plan_substep(tmpm_session* s, bool apply_force) {
   SubstepPlan pl;
   std::memset(&pl, 0, sizeof pl);
   pl.p = s->parts(s->cur);
-  pl.reorder = s->substeps_since_reorder >= s->reorder_interval;
+  const bool may_list = !s->cpic;
+  pl.reorder = s->substeps_since_reorder >= s->reorder_interval ||
+               (may_list && !s->lists_valid && s->reorder_interval > 1 && s->reorder_interval <= kListSpan);
   if (pl.reorder) pl.q = s->parts(1 - s->cur);
   pl.t = s->topo;
+  const bool listed = !pl.reorder && may_list && s->lists_valid;
+  const uint32_t since = pl.reorder ? 1u : s->substeps_since_reorder + 1;  // after this substep
+  const bool build = may_list && (pl.reorder || listed) && since < s->reorder_interval && since < kListSpan;
+  pl.t.listed = listed ? 1 : 0;
+  pl.t.build = build ? 1 : 0;
+  const int read = listed ? s->list_read : 0;
+  pl.t.cur = block_lists(s, read);
+  if (!listed) {
+    pl.t.cur.idx = s->topo.sorted;
+    pl.t.cur.pitch = 0;
+  }
+  pl.t.nxt = block_lists(s, 1 - read);
   pl.c = s->classes.as<DevClass>();
   pl.sc = (apply_force ? s->scene_force : s->scene_plain).as<DevScene>();
   pl.sc_plain = s->scene_plain.as<DevScene>();
@@ -1942,7 +1994,7 @@ SubstepPlan plan_substep(tmpm_session* s, bool apply_force) {
   pl.shapes = s->shapes;
   pl.plastic = s->plastic ? 1 : 0;
   pl.cpic = s->cpic;
-  pl.clear_table = s->table_dirty;
+  pl.clear_table = s->table_dirty && !listed;
   pl.rigid_sync = s->body_total > 0 && s->obstacle_total > 0;
   pl.rigid_apply = pl.react && s->body_total > 0;
   pl.audit = s->audit_on ? s->audit_next : nullptr;
@@ -1964,15 +2016,20 @@ hipError_t launch_plan(tmpm_session* s, const SubstepPlan& pl) {
   if (pl.cpic &&
       (e = timed(s, "k_cpic_mask", [&] { launch_cpic_mask(p, t, pl.c, pl.sc_plain, pl.ob, st); })) != hipSuccess)
     return e;
-  if ((e = timed(s, "k_bin_insert", [&] { launch_bin_insert(p, t, pl.c, pl.sc_plain, pl.cpic, st); })) !=
-      hipSuccess)
-    return e;
-  if ((e = timed(s, "k_bin_blocks", [&] { launch_bin_blocks(p, t, pl.c, pl.sc_plain, pl.cpic, st); })) !=
-      hipSuccess)
-    return e;
-  if ((e = timed(s, "k_bin_offsets", [&] { launch_bin_offsets(p, t, pl.c, pl.sc_plain, st); })) != hipSuccess)
-    return e;
-  if ((e = timed(s, "k_bin_scatter", [&] { launch_bin_scatter(p, t, st); })) != hipSuccess) return e;
+  if (t.listed) {
+    if ((e = timed(s, "k_bin_update", [&] { launch_bin_update(p, t, pl.c, pl.sc_plain, st); })) != hipSuccess)
+      return e;
+  } else {
+    if ((e = timed(s, "k_bin_insert", [&] { launch_bin_insert(p, t, pl.c, pl.sc_plain, pl.cpic, st); })) !=
+        hipSuccess)
+      return e;
+    if ((e = timed(s, "k_bin_blocks", [&] { launch_bin_blocks(p, t, pl.c, pl.sc_plain, pl.cpic, st); })) !=
+        hipSuccess)
+      return e;
+    if ((e = timed(s, "k_bin_offsets", [&] { launch_bin_offsets(p, t, pl.c, pl.sc_plain, st); })) != hipSuccess)
+      return e;
+    if ((e = timed(s, "k_bin_scatter", [&] { launch_bin_scatter(p, t, st); })) != hipSuccess) return e;
+  }
   if ((e = timed(s, pl.fixed64 ? "k_p2g_fixed64" : "k_p2g", [&] {
          launch_p2g(p, t, pl.c, pl.sc, pl.fixed64, pl.p2g_blocks, pl.p2g_threads, pl.copies, pl.plastic, st);
        })) != hipSuccess)
@@ -2002,7 +2059,7 @@ hipError_t launch_plan(tmpm_session* s, const SubstepPlan& pl) {
 // Replays the graph captured for an equal plan, or captures one.  At most
 // kGraphCache graphs are kept (least recently used evicted): a steady run
 // cycles through a few plans (buffer parity, reorder or not).
-constexpr size_t kGraphCache = 8;
+constexpr size_t kGraphCache = 16;
 
 hipError_t launch_graph(tmpm_session* s, const SubstepPlan& pl) {
   for (auto& g : s->graphs)
@@ -2050,7 +2107,9 @@ hipError_t enqueue_substep(tmpm_session* s, bool apply_force) {
   if ((uint64_t)pl.t.bin_groups * pl.t.bin_span < pl.p.n) return hipErrorInvalidValue;  // lists sized for fewer particles
   const hipError_t e = s->use_graphs && !s->timing && !pl.audit ? launch_graph(s, pl) : launch_plan(s, pl);
   if (e != hipSuccess) return e;
-  if (pl.clear_table) s->table_dirty = false;
+  s->lists_valid = pl.t.build != 0;
+  s->list_read = pl.t.listed ? 1 - s->list_read : 1;
+  s->table_dirty = pl.t.build != 0;  // otherwise G2P cleared the block table
   if (pl.reorder) {
     s->compacted_last = true;
     s->cur = 1 - s->cur;
@@ -2891,6 +2950,7 @@ tmpm_status commit_staged(tmpm_session* s, tmpm_staged_scene& staged, uint32_t* 
     swap_bufs(s->synced, synced);
     s->cap = cap;
   }
+  s->lists_valid = false;  // the new particles are on no list
   if ((st = upload_particles(s, pk, s->n)) != TMPM_OK) return broken(st);
   s->n += (uint32_t)pk.size();
   s->n_enabled = s->n;
@@ -3132,6 +3192,7 @@ tmpm_status tmpm_session_synchronize(tmpm_session* s) {
         scene.status = status_from_error_bits(scene_bits[k]);  // the last synchronized world stays readable
         stopped = true;
         if (s->prepared && scene.count) {
+          s->lists_valid = false;  // its particles leave their blocks' ranges and lists
           launch_retire(s->parts(s->cur), scene.first, scene.count, s->stream);
           HIP_TRY(hipGetLastError());
         }
@@ -3511,6 +3572,7 @@ tmpm_status tmpm_batch_remove_scene(tmpm_session* s, uint32_t scene) {
       // next reorder drops them) and the insertion indices above its range
       // close the gap, here and in the synchronized copy.
       Parts p = s->parts(s->cur);
+      s->lists_valid = false;
       launch_retire(p, first, count, s->stream);
       launch_renumber(p.ins_id, s->n, first, count, s->stream);
       launch_renumber(s->synced.ins_id.as<uint32_t>(), s->synced_n, first, count, s->stream);

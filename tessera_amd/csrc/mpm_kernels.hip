@@ -2796,15 +2796,101 @@ __global__ __launch_bounds__(256) void k_live_count(Topo t) {
 // ---------------------------------------------------------------------------
 // Closed-mesh volume sampling (sampling.rs:47-146): lattice centres whose
 // solid angle subtended by the mesh exceeds 2 pi (winding number 1, either
-// orientation).  One thread per candidate, f64 throughout, triangles in the
-// reference's order; flags[c] = 1 for an accepted candidate.
+// orientation), f64 throughout; flags[c] = 1 for an accepted candidate.
+//
+// k_mesh_winding decides all candidates that are clear of the surface.  A
+// triangle's angle is that of the complex number (den, num), and the angle of
+// a product is the sum of the angles up to whole turns, which the signs of the
+// imaginary parts count: one complex product per triangle in place of an
+// atan2.  The triangles are split over the `waves` wavefronts of a workgroup
+// (64 candidates, one per lane; the triangle is uniform, so its vertices are
+// scalar loads), which fills the chip where the lattice is small.  The sum is
+// a whole number of turns, so it is decided by a margin of pi; where a
+// triangle's number is next to zero or to the negative real axis (the
+// candidate lies on the surface, or the mesh's scale over- or underflows), the
+// candidate is left to k_mesh_inside, one thread per candidate that sums the
+// angles in the reference's order.
+// Bound by f64 issue (75 f64 operations per pair).  1,280 triangles and 18,400
+// candidates: 137 us, and 4 us for k_mesh_inside over the undecided ones; 704 us
+// with an atan2 per pair on one thread per candidate (72 workgroups).
 // ---------------------------------------------------------------------------
+constexpr uint8_t kMeshUndecided = 2;
+
+// sqrt(x) to ~1e-15 for normal x > 0; NaN at 0
+__device__ __forceinline__ double mesh_root(double x) {
+  const double y = __builtin_amdgcn_rsq(x), r = x * y;
+  return __builtin_fma(0.5 * y, __builtin_fma(-r, r, x), r);
+}
+
+__global__ __launch_bounds__(1024) void k_mesh_winding(const double* __restrict__ verts,
+                                                       const uint32_t* __restrict__ tris, uint64_t ntri, double lx,
+                                                       double ly, double lz, double spacing, uint64_t cy, uint64_t cz,
+                                                       double ux, double uy, double uz, uint64_t count,
+                                                       uint8_t* flags) {
+  __shared__ double s_angle[16][64];
+  __shared__ uint32_t s_near[16][64];
+  const uint32_t lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint64_t t0 = ntri * wave / waves, t1 = ntri * (wave + 1) / waves;
+  for (uint64_t c0 = (uint64_t)blockIdx.x * 64; c0 < count; c0 += (uint64_t)gridDim.x * 64) {
+    const uint64_t c = c0 + lane;
+    const uint64_t x = c / (cy * cz), y = (c / cz) % cy, z = c % cz;
+    const double px = lx + ((double)x + 0.5) * spacing;
+    const double py = ly + ((double)y + 0.5) * spacing;
+    const double pz = lz + ((double)z + 0.5) * spacing;
+    double re = 1.0, im = 0.0;
+    int turns = 0;
+    bool near = false;
+#pragma unroll 2
+    for (uint64_t t = t0; t < t1; ++t) {
+      double v[3][3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double* q = verts + 3ull * tris[3 * t + k];
+        v[k][0] = q[0] - px;
+        v[k][1] = q[1] - py;
+        v[k][2] = q[2] - pz;
+      }
+      auto dot = [](const double* a, const double* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; };
+      const double la = mesh_root(dot(v[0], v[0])), lb = mesh_root(dot(v[1], v[1])), lc = mesh_root(dot(v[2], v[2]));
+      const double bc[3] = {v[1][1] * v[2][2] - v[1][2] * v[2][1], v[1][2] * v[2][0] - v[1][0] * v[2][2],
+                            v[1][0] * v[2][1] - v[1][1] * v[2][0]};
+      const double num = dot(v[0], bc), size = la * lb * lc;
+      const double den = size + dot(v[0], v[1]) * lc + dot(v[1], v[2]) * la + dot(v[2], v[0]) * lb;
+      const double tiny = 1e-9 * size;
+      near |= !(size > 1e-280 && size < 1e280) || !(fabs(num) > tiny || den > tiny);
+      const double r = re * den - im * num, i = re * num + im * den;
+      turns += im >= 0.0 && num >= 0.0 && i < 0.0 ? 1 : im < 0.0 && num < 0.0 && i >= 0.0 ? -1 : 0;
+      const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(r), fabs(i)));
+      re = __builtin_ldexp(r, e);
+      im = __builtin_ldexp(i, e);
+    }
+    s_angle[wave][lane] = 6.283185307179586 * turns + atan2(im, re);
+    s_near[wave][lane] = near;
+    __syncthreads();
+    if (wave == 0 && c < count) {
+      double angle = 0.0;
+      uint32_t undecided = 0;
+      for (uint32_t w = 0; w < waves; ++w) {
+        angle += s_angle[w][lane];
+        undecided |= s_near[w][lane];
+      }
+      const double a = fabs(angle);
+      const bool out = px >= ux || py >= uy || pz >= uz;
+      flags[c] = out ? 0 : undecided || !(fabs(a - 3.141592653589793) > 1.0) ? kMeshUndecided : a > 3.141592653589793;
+    }
+    __syncthreads();
+  }
+}
+
+// The candidates that k_mesh_winding left undecided.
 __global__ __launch_bounds__(256) void k_mesh_inside(const double* __restrict__ verts,
                                                      const uint32_t* __restrict__ tris, uint64_t ntri,
                                                      double lx, double ly, double lz, double spacing, uint64_t cy,
                                                      uint64_t cz, double ux, double uy, double uz, uint64_t count,
                                                      uint8_t* flags) {
   for (uint64_t c = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; c < count; c += (uint64_t)gridDim.x * blockDim.x) {
+    if (flags[c] != kMeshUndecided) continue;
     const uint64_t x = c / (cy * cz), y = (c / cz) % cy, z = c % cz;
     const double px = lx + ((double)x + 0.5) * spacing;
     const double py = ly + ((double)y + 0.5) * spacing;
@@ -3041,6 +3127,13 @@ void launch_mesh_inside(const double* verts, const uint32_t* tris, uint64_t ntri
                         const double upper[3], double spacing, const uint64_t counts[3], uint8_t* flags,
                         hipStream_t s) {
   const uint64_t count = counts[0] * counts[1] * counts[2];
+  // Wavefronts per workgroup, which share its 64 candidates' triangles: 16 until
+  // that makes 64 waves per SIMD, and at least 8 triangles each.
+  uint32_t waves = 16;
+  while (waves > 1 && (waves * ((count + 63) / 64) > 65536 || ntri < 8ull * waves)) waves /= 2;
+  hipLaunchKernelGGL(k_mesh_winding, dim3(grid_for(count, 64, 1u << 20)), dim3(64 * waves), 0, s, verts, tris, ntri,
+                     lower[0], lower[1], lower[2], spacing, counts[1], counts[2], upper[0], upper[1], upper[2], count,
+                     flags);
   hipLaunchKernelGGL(k_mesh_inside, dim3(grid_for(count, 256, 65536)), dim3(256), 0, s, verts, tris, ntri, lower[0],
                      lower[1], lower[2], spacing, counts[1], counts[2], upper[0], upper[1], upper[2], count, flags);
 }

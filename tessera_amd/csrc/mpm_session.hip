@@ -2449,6 +2449,42 @@ struct MeshLattice {
   uint64_t candidates;
 };
 
+// sampling.rs:66-93: every undirected edge used exactly once in each direction
+// (a closed, consistently oriented surface).  Open-addressed table of the
+// undirected edges, with a bit for each direction seen.
+bool mesh_closed(const uint32_t* triangles, uint64_t triangle_count) {
+  struct Edge {
+    uint32_t a, b;  // a < b; a == b: empty
+    uint32_t seen;
+  };
+  const uint64_t edges = 3 * triangle_count;
+  uint64_t size = 64;
+  while (size < 2 * edges) size *= 2;
+  std::vector<Edge> table(size, Edge{0, 0, 0});
+  uint64_t used = 0, done = 0;
+  for (uint64_t t = 0; t < triangle_count; ++t)
+    for (int k = 0; k < 3; ++k) {
+      const uint32_t p = triangles[3 * t + k], q = triangles[3 * t + (k + 1) % 3];
+      const uint32_t a = std::min(p, q), b = std::max(p, q), bit = p > q ? 2u : 1u;
+      uint64_t h = (((uint64_t)a << 32) | b) * 0x9E3779B97F4A7C15ull;
+      h ^= h >> 29;
+      for (h &= size - 1;; h = (h + 1) & (size - 1)) {
+        Edge& e = table[h];
+        if (e.a == e.b) {
+          e = Edge{a, b, bit};
+          ++used;
+          break;
+        }
+        if (e.a != a || e.b != b) continue;
+        if (e.seen & bit) return false;
+        e.seen |= bit;
+        ++done;
+        break;
+      }
+    }
+  return used == done;  // each edge seen in the second direction too
+}
+
 // sampling.rs:94-115: the AABB lattice, bounded by max_candidates.
 tmpm_status mesh_lattice(const double* vertices, uint64_t vertex_count, double spacing, uint64_t max_candidates,
                          MeshLattice& lat) {
@@ -2475,15 +2511,22 @@ tmpm_status mesh_lattice(const double* vertices, uint64_t vertex_count, double s
 // to samples_out in lattice order (x, then y, then z), at most max_samples.
 tmpm_status mesh_emit_samples(const MeshLattice& lat, double spacing, const uint8_t* flags, uint64_t c0,
                               uint64_t len, uint64_t max_samples, double* samples_out, uint64_t& n) {
-  for (uint64_t c = c0; c < c0 + len; ++c) {
-    if (!flags[c - c0]) continue;
-    if (n == max_samples) return fail(TMPM_CAPACITY, "accepted samples exceed max_samples");
-    const uint64_t x = c / (lat.counts[1] * lat.counts[2]), y = (c / lat.counts[2]) % lat.counts[1],
-                   z = c % lat.counts[2];
-    samples_out[3 * n] = lat.lower[0] + ((double)x + 0.5) * spacing;
-    samples_out[3 * n + 1] = lat.lower[1] + ((double)y + 0.5) * spacing;
-    samples_out[3 * n + 2] = lat.lower[2] + ((double)z + 0.5) * spacing;
-    ++n;
+  uint64_t x = c0 / (lat.counts[1] * lat.counts[2]), y = (c0 / lat.counts[2]) % lat.counts[1], z = c0 % lat.counts[2];
+  for (uint64_t c = 0; c < len; ++c) {
+    if (flags[c]) {
+      if (n == max_samples) return fail(TMPM_CAPACITY, "accepted samples exceed max_samples");
+      samples_out[3 * n] = lat.lower[0] + ((double)x + 0.5) * spacing;
+      samples_out[3 * n + 1] = lat.lower[1] + ((double)y + 0.5) * spacing;
+      samples_out[3 * n + 2] = lat.lower[2] + ((double)z + 0.5) * spacing;
+      ++n;
+    }
+    if (++z == lat.counts[2]) {
+      z = 0;
+      if (++y == lat.counts[1]) {
+        y = 0;
+        ++x;
+      }
+    }
   }
   return TMPM_OK;
 }
@@ -4104,38 +4147,57 @@ tmpm_status tmpm_sample_closed_mesh_volume(tmpm_context* ctx, const double* vert
     tmpm_status st = mesh_check_triangles(ctx, vertices, vertex_count, triangles, triangle_count, spacing,
                                           max_candidates, max_samples, samples_out, count_out);
     if (st != TMPM_OK) return st;
-    // sampling.rs:66-93: every undirected edge used exactly once in each
-    // direction (a closed, consistently oriented surface)
-    std::map<std::pair<uint32_t, uint32_t>, std::array<uint64_t, 2>> edges;
-    for (uint64_t t = 0; t < triangle_count; ++t) {
-      const uint32_t* tr = triangles + 3 * t;
-      const uint32_t pairs[3][2] = {{tr[0], tr[1]}, {tr[1], tr[2]}, {tr[2], tr[0]}};
-      for (const auto& pr : pairs)
-        edges[{std::min(pr[0], pr[1]), std::max(pr[0], pr[1])}][pr[0] > pr[1] ? 1 : 0] += 1;
-    }
-    for (const auto& e : edges)
-      if (e.second[0] != 1 || e.second[1] != 1)
-        return fail(TMPM_INVALID_INPUT, "mesh is not closed and consistently oriented");
     MeshLattice lat;
-    if ((st = mesh_lattice(vertices, vertex_count, spacing, max_candidates, lat)) != TMPM_OK) return st;
-    // sampling.rs:116-144 on the device: the solid-angle test of every candidate
+    const bool fits = mesh_lattice(vertices, vertex_count, spacing, max_candidates, lat) == TMPM_OK;
+    if (!fits) {
+      if (!mesh_closed(triangles, triangle_count))
+        return fail(TMPM_INVALID_INPUT, "mesh is not closed and consistently oriented");
+      return mesh_lattice(vertices, vertex_count, spacing, max_candidates, lat);
+    }
+    // sampling.rs:116-144 on the device: the solid-angle test of every
+    // candidate, in the fixed scratch of the device if it is free and large
+    // enough.  The host tests the edges meanwhile.
     if (hipSetDevice(ctx->device) != hipSuccess) return fail(TMPM_NO_DEVICE, "cannot select device");
-    DevBuf dv, dt, df;
-    HIP_TRY(dv.alloc(24ull * vertex_count));
-    HIP_TRY(dt.alloc(12ull * triangle_count));
-    HIP_TRY(df.alloc(lat.candidates));
-    HIP_TRY(hipMemcpy(dv.ptr, vertices, 24ull * vertex_count, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dt.ptr, triangles, 12ull * triangle_count, hipMemcpyHostToDevice));
-    hipStream_t stream = nullptr;
-    HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-    launch_mesh_inside(dv.as<double>(), dt.as<uint32_t>(), triangle_count, lat.lower, lat.upper, spacing, lat.counts,
-                       df.as<uint8_t>(), stream);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
-    (void)hipStreamDestroy(stream);
-    if (e != hipSuccess) return fail(TMPM_READBACK, std::string("mesh sampling kernel failed: ") + hipGetErrorString(e));
+    const uint64_t off_t = 24ull * vertex_count, off_f = off_t + 12ull * triangle_count;
+    NoAllocScratch& ns = noalloc_scratch(ctx->device);
+    std::unique_lock<std::mutex> lock(ns.mu, std::defer_lock);
+    DevBuf own;
+    char* base = nullptr;
+    if (off_f + lat.candidates <= kScratchBytes && ns.ptr && lock.try_lock()) {
+      base = static_cast<char*>(ns.ptr);
+    } else {
+      HIP_TRY(own.alloc(off_f + lat.candidates));
+      base = static_cast<char*>(own.ptr);
+    }
+    std::vector<char> mesh(off_f);
+    std::memcpy(mesh.data(), vertices, off_t);
+    std::memcpy(mesh.data() + off_t, triangles, 12ull * triangle_count);
     std::vector<uint8_t> flags(lat.candidates);
-    HIP_TRY(hipMemcpy(flags.data(), df.ptr, lat.candidates, hipMemcpyDeviceToHost));
+    struct Stream {
+      hipStream_t s = nullptr;
+      ~Stream() {
+        if (s) (void)hipStreamDestroy(s);
+      }
+    } stream;
+    HIP_TRY(hipStreamCreateWithFlags(&stream.s, hipStreamNonBlocking));
+    HIP_TRY(hipMemcpyAsync(base, mesh.data(), off_f, hipMemcpyHostToDevice, stream.s));
+    launch_mesh_inside(reinterpret_cast<const double*>(base), reinterpret_cast<const uint32_t*>(base + off_t),
+                       triangle_count, lat.lower, lat.upper, spacing, lat.counts, reinterpret_cast<uint8_t*>(base + off_f),
+                       stream.s);
+    hipError_t e = hipGetLastError();
+    bool closed = false, threw = false;
+    try {
+      closed = mesh_closed(triangles, triangle_count);
+    } catch (...) {
+      threw = true;  // the device still reads the buffers
+    }
+    if (e == hipSuccess && closed)
+      e = hipMemcpyAsync(flags.data(), base + off_f, lat.candidates, hipMemcpyDeviceToHost, stream.s);
+    const hipError_t w = hipStreamSynchronize(stream.s);
+    if (e == hipSuccess) e = w;
+    if (threw) return fail(TMPM_CAPACITY, "host memory exhausted");
+    if (e != hipSuccess) return fail(TMPM_READBACK, std::string("mesh sampling kernel failed: ") + hipGetErrorString(e));
+    if (!closed) return fail(TMPM_INVALID_INPUT, "mesh is not closed and consistently oriented");
     uint64_t n = 0;
     if ((st = mesh_emit_samples(lat, spacing, flags.data(), 0, lat.candidates, max_samples, samples_out, n)) != TMPM_OK)
       return st;

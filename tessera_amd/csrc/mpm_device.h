@@ -122,8 +122,9 @@ struct DevObstacle {
   int32_t cpic_group;    // -1: none
   int32_t pad4[3];
 };
-constexpr int kMaxConvexPlanes = 128;
-constexpr int kGatherFloats = 29;  // per particle in a scene gather (k_gather_scene)  // planes per convex obstacle (gpu.rs pack_obstacle)
+constexpr int kMaxConvexPlanes = 128;  // planes per convex obstacle (gpu.rs pack_obstacle)
+constexpr int kGatherFloats = 29;    // per particle in a scene gather (k_gather_scene)
+constexpr int kReadbackHeader = 16;  // words before the records of k_gather_state
 
 // Rigid body state (GpuRigidBodyState, phys/src/gpu_rigid_state.rs:17-28):
 // position and inverse mass, XYZW orientation, world velocities, body-frame

@@ -2671,22 +2671,49 @@ __global__ __launch_bounds__(256) void k_renumber(uint32_t* ins_id, uint32_t n, 
 // One scene's particles in insertion order, kGatherFloats each: x, y, z,
 // mass, vx, vy, vz, volume, C (9, column-major), F (9), plastic state (3;
 // 1, 0, 0 when the session stores none).
+__device__ __forceinline__ void gather_record(const Parts& p, uint32_t i, float* r, bool& finite) {
+  r[26] = p.P ? p.P[i] : 1.0f;
+  r[27] = p.P ? p.P[p.stride + i] : 0.0f;
+  r[28] = p.P ? p.P[2 * p.stride + i] : 0.0f;
+  const float4 a = p.pos_mass[i], b = p.vel_vol[i];
+  r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
+  r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
+  auto fin = [](float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; };
+  finite = fin(a.x) && fin(a.y) && fin(a.z) && fin(b.x) && fin(b.y) && fin(b.z);
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    const float c = p.C[q * p.stride + i], f = p.F[q * p.stride + i];
+    r[8 + q] = c;
+    r[17 + q] = f;
+    finite = finite && fin(c) && fin(f);
+  }
+}
+
 __global__ __launch_bounds__(256) void k_gather_scene(Parts p, uint32_t first, uint32_t count, float* out) {
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < p.n; i += gridDim.x * blockDim.x) {
     const uint32_t g = p.ins_id[i];
     if (g == kInvalid || g - first >= count) continue;
-    float* r = out + (size_t)(g - first) * kGatherFloats;
-    r[26] = p.P ? p.P[i] : 1.0f;
-    r[27] = p.P ? p.P[p.stride + i] : 0.0f;
-    r[28] = p.P ? p.P[2 * p.stride + i] : 0.0f;
-    const float4 a = p.pos_mass[i], b = p.vel_vol[i];
-    r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
-    r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-      r[8 + q] = p.C[q * p.stride + i];
-      r[17 + q] = p.F[q * p.stride + i];
-    }
+    bool finite;
+    gather_record(p, i, out + (size_t)(g - first) * kGatherFloats, finite);
+  }
+}
+
+// A plain session's readback: kReadbackHeader words (the counters, the scene's
+// error bits, and `mark` in the last one if a particle that moves is not
+// finite), then every particle's record by insertion index, in one buffer for
+// one copy to the host.
+__global__ __launch_bounds__(256) void k_gather_state(Parts p, const DevClass* classes, const uint32_t* counters,
+                                                      const uint32_t* scene_err, uint32_t mark, uint32_t count,
+                                                      float* out) {
+  uint32_t* header = reinterpret_cast<uint32_t*>(out);
+  if (blockIdx.x == 0 && threadIdx.x < CNT_COUNT) header[threadIdx.x] = counters[threadIdx.x];
+  if (blockIdx.x == 0 && threadIdx.x == CNT_COUNT) header[CNT_COUNT] = scene_err[0];
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < p.n; i += gridDim.x * blockDim.x) {
+    const uint32_t g = p.ins_id[i];
+    if (g >= count) continue;  // kInvalid: no particle in the slot
+    bool finite;
+    gather_record(p, i, out + kReadbackHeader + (size_t)g * kGatherFloats, finite);
+    if (!finite && !classes[p.cls[i]].fixed) header[kReadbackHeader - 1] = mark;
   }
 }
 
@@ -3113,6 +3140,11 @@ void launch_renumber(uint32_t* ins_id, uint32_t n, uint32_t first, uint32_t coun
 }
 void launch_gather_scene(const Parts& p, uint32_t first, uint32_t count, float* out, hipStream_t s) {
   hipLaunchKernelGGL(k_gather_scene, dim3(grid_for(p.n, 256, 8192)), dim3(256), 0, s, p, first, count, out);
+}
+void launch_gather_state(const Parts& p, const DevClass* c, const Topo& t, uint32_t mark, uint32_t count, float* out,
+                         hipStream_t s) {
+  hipLaunchKernelGGL(k_gather_state, dim3(grid_for(p.n, 256, 8192)), dim3(256), 0, s, p, c, t.counters, t.scene_err, mark,
+                     count, out);
 }
 void launch_audit(const Parts& p, const DevClass* c, double* out, hipStream_t s) {
   hipLaunchKernelGGL(k_audit, dim3(grid_for(p.n, 256, 4096)), dim3(256), 0, s, p, c, out);

@@ -626,6 +626,7 @@ struct tmpm_session {
   ParticleBuffers synced;
   uint32_t synced_n = 0;
   DevBuf staging;
+  uint32_t readback_mark = 0;
   DevBuf disabled_rec;     // snapshot records of disabled particles (2 float4 each)
   std::vector<float4> disabled_host;
   PackedParticles stage;                // admission staging, reused
@@ -2169,72 +2170,150 @@ tmpm_status status_from_error_bits(uint32_t bits) {
   return TMPM_OK;
 }
 
-// Copies device state into new worlds (gpu.rs:2295-2329 apply_gpu_transfers):
-// out[k] is scene k's updated world and st[k] TMPM_NON_FINITE_STATE if one of
-// its particles is not finite.  Scenes that are not stepping are left as is.
-tmpm_status read_back(tmpm_session* s, std::vector<HostWorld>& out, std::vector<tmpm_status>& st) {
-  const size_t ns = s->scenes.size();
-  out.assign(ns, HostWorld());
-  st.assign(ns, TMPM_OK);
-  for (size_t k = 0; k < ns; ++k) {
-    if (!s->scenes[k].stepping()) continue;
-    HostWorld& w = out[k];
-    w = s->scenes[k].world;
-    // forces are one-shot; fixed particles end with zero v and C (world.rs:419-430)
-    for (size_t i = 0; i < w.size(); ++i) {
+// Page-locked readback buffers, reused by every session of the process:
+// page-locking costs more than most readbacks.  At most kKept buffers of at
+// most kBytes are kept; any thread may take and give back.
+struct ReadbackPool {
+  static constexpr size_t kBytes = 16u << 20, kKept = 8;
+  struct Buffer {
+    PodBuf<float, true> mem;
+    int device = 0;
+    hipEvent_t copied = nullptr;  // of that device
+    ~Buffer() {
+      if (copied) (void)hipEventDestroy(copied);
+    }
+  };
+  std::mutex mu;
+  std::vector<std::unique_ptr<Buffer>> free_;
+  // `device` is current
+  std::unique_ptr<Buffer> acquire(int device, size_t floats) {
+    {
+      std::lock_guard<std::mutex> lock(mu);
+      for (size_t i = free_.size(); i-- > 0;)
+        if (free_[i]->device == device && free_[i]->mem.cap >= floats) {
+          std::unique_ptr<Buffer> b = std::move(free_[i]);
+          free_.erase(free_.begin() + i);
+          b->mem.resize(floats);
+          return b;
+        }
+    }
+    std::unique_ptr<Buffer> b(new Buffer());
+    b->mem.resize(next_pow2(floats));
+    b->mem.resize(floats);
+    b->device = device;
+    if (hipEventCreateWithFlags(&b->copied, hipEventDisableTiming) != hipSuccess) throw std::bad_alloc();
+    return b;
+  }
+  void release(std::unique_ptr<Buffer> b) {
+    if (!b) return;
+    std::lock_guard<std::mutex> lock(mu);
+    if (free_.size() >= kKept) free_.erase(free_.begin());
+    free_.push_back(std::move(b));
+  }
+};
+
+ReadbackPool& readback_pool() {
+  static ReadbackPool* p = new ReadbackPool();  // never destroyed: the HIP runtime may be gone by then
+  return *p;
+}
+
+// The buffers of one readback, given back when it ends.
+struct ReadbackBuffers {
+  std::unique_ptr<ReadbackPool::Buffer> b[2];
+  ~ReadbackBuffers() {
+    for (auto& p : b) readback_pool().release(std::move(p));
+  }
+};
+
+// Records [first, first + count) of a k_gather_state buffer into the world
+// (gpu.rs:2295-2329 apply_gpu_transfers): f32 widened to f64.  Forces are
+// one-shot; fixed particles end with zero v and C (world.rs:419-430).
+void widen_records(HostWorld& w, const float* rec, size_t first, size_t count, bool records, bool plastic) {
+  parallel_for(count, [&](size_t b, size_t e) {
+    for (size_t k = b; k < e; ++k) {
+      const size_t i = first + k;
       w.force[3 * i] = w.force[3 * i + 1] = w.force[3 * i + 2] = 0.0;
-      if (w.fixed[i] && w.enabled[i]) {
+      if (!w.enabled[i]) continue;
+      if (w.fixed[i]) {
         for (int q = 0; q < 3; ++q) w.vel[3 * i + q] = 0.0;
         for (int q = 0; q < 9; ++q) w.C[9 * i + q] = 0.0;
+        continue;
       }
+      if (!records) continue;
+      const float* r = rec + k * kGatherFloats;
+      for (int q = 0; q < 3; ++q) {
+        w.pos[3 * i + q] = r[q];
+        w.vel[3 * i + q] = r[4 + q];
+      }
+      for (int q = 0; q < 9; ++q) {
+        w.C[9 * i + q] = r[8 + q];
+        w.F[9 * i + q] = r[17 + q];
+      }
+      if (plastic && is_plastic(w.material[i]))
+        for (int q = 0; q < 3; ++q) w.plastic[3 * i + q] = r[26 + q];
     }
+  });
+}
+
+// A plain session's readback: one kernel lays the counters and every
+// particle's record out in insertion order, one copy (in pieces, of which the
+// host widens one while the next is copied) brings them to page-locked memory.
+// `check` sees the counters and scene error bits before the world is touched;
+// a status other than TMPM_OK ends the readback.  The host spent 8.2 ms on
+// 59,319 particles with a copy per column, two copies of the world and a
+// serial scatter.
+template <class F>
+tmpm_status read_back(tmpm_session* s, uint32_t counters[CNT_COUNT], F&& check) {
+  SceneState& scene = s->scenes[0];
+  HostWorld& w = scene.world;
+  if (!s->prepared) {
+    tmpm_status st = check(0u, false);
+    if (st == TMPM_OK) widen_records(w, nullptr, 0, w.size(), false, false);
+    return st;
   }
-  if (!s->prepared) return TMPM_OK;
-  size_t n = s->n;
-  const ParticleBuffers& b = s->buf[s->cur];
-  std::vector<float4> pm(n), vv(n);
-  std::vector<float> C(9 * n), F(9 * n);
-  std::vector<uint32_t> ins(n);
-  HIP_TRY(hipMemcpy(pm.data(), b.pos_mass.ptr, 16 * n, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(vv.data(), b.vel_vol.ptr, 16 * n, hipMemcpyDeviceToHost));
-  for (int q = 0; q < 9; ++q) {
-    HIP_TRY(hipMemcpy(C.data() + (size_t)q * n, b.C.as<float>() + (size_t)q * s->cap, 4 * n, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(F.data() + (size_t)q * n, b.F.as<float>() + (size_t)q * s->cap, 4 * n, hipMemcpyDeviceToHost));
-  }
-  HIP_TRY(hipMemcpy(ins.data(), b.ins_id.ptr, 4 * n, hipMemcpyDeviceToHost));
-  std::vector<float> P(s->plastic ? 3 * n : 0);
-  for (int q = 0; q < 3 && s->plastic; ++q)
-    HIP_TRY(hipMemcpy(P.data() + (size_t)q * n, b.P.as<float>() + (size_t)q * s->cap, 4 * n, hipMemcpyDeviceToHost));
-  // insertion index -> scene: scenes occupy consecutive ranges
-  std::vector<std::pair<uint32_t, uint32_t>> ranges;  // (first, scene)
-  for (uint32_t k = 0; k < ns; ++k)
-    if (s->scenes[k].count) ranges.emplace_back(s->scenes[k].first, k);
-  for (size_t slot = 0; slot < n; ++slot) {
-    const uint32_t g = ins[slot];
-    if (g == kInvalid) continue;  // retired slot
-    auto it = std::upper_bound(ranges.begin(), ranges.end(), std::make_pair(g, UINT32_MAX));
-    if (it == ranges.begin()) return fail(TMPM_READBACK, "corrupt particle order");
-    const uint32_t k = (it - 1)->second;
-    const size_t i = g - s->scenes[k].first;
-    HostWorld& w = out[k];
-    if (i >= w.size() || i >= s->scenes[k].count) return fail(TMPM_READBACK, "corrupt particle order");
-    if (!w.enabled[i] || w.fixed[i]) continue;
-    const float4 p = pm[slot], v = vv[slot];
-    double xs[3] = {p.x, p.y, p.z}, vs[3] = {v.x, v.y, v.z};
-    bool finite = true;
-    for (int q = 0; q < 3; ++q) {
-      w.pos[3 * i + q] = xs[q];
-      w.vel[3 * i + q] = vs[q];
-      finite = finite && std::isfinite(xs[q]) && std::isfinite(vs[q]);
+  if (hipSetDevice(s->ctx->device) != hipSuccess) return fail(TMPM_READBACK, "cannot select device");
+  const size_t n = scene.count, words = kReadbackHeader + n * kGatherFloats;
+  if (s->staging.bytes < 4 * words) HIP_TRY(s->staging.alloc(4 * words));
+  const uint32_t mark = ++s->readback_mark | 0x80000000u;
+  float* dev = s->staging.as<float>();
+  launch_gather_state(s->parts(s->cur), s->classes.as<DevClass>(), s->topo, mark, (uint32_t)n, dev,
+                      s->stream);
+  HIP_TRY(hipGetLastError());
+  // pieces of whole records; the first one has the header
+  const size_t per = (ReadbackPool::kBytes / 4 - kReadbackHeader) / kGatherFloats;
+  const size_t pieces = std::max<size_t>(1, (n + per - 1) / per);
+  ReadbackBuffers buf;
+  for (size_t k = 0; k < std::min<size_t>(2, pieces); ++k)
+    buf.b[k] = readback_pool().acquire(s->ctx->device, kReadbackHeader + std::min(n, per) * kGatherFloats);
+  auto copy = [&](size_t k) -> hipError_t {
+    const size_t from = k * per, count = std::min(n - from, per), head = k == 0 ? kReadbackHeader : 0;
+    ReadbackPool::Buffer& b = *buf.b[k & 1];
+    hipError_t e = hipMemcpyAsync(b.mem.data(), dev + (k == 0 ? 0 : kReadbackHeader + from * kGatherFloats),
+                                  4 * (head + count * kGatherFloats), hipMemcpyDeviceToHost, s->stream);
+    return e == hipSuccess ? hipEventRecord(b.copied, s->stream) : e;
+  };
+  // a copy in flight ends before its buffer goes back to the pool
+  struct Drain {
+    hipStream_t s;
+    ~Drain() { (void)hipStreamSynchronize(s); }
+  };
+  {
+    Drain drain{s->stream};
+    hipError_t e = copy(0);
+    for (size_t k = 0; k < pieces; ++k) {
+      if (e == hipSuccess && k + 1 < pieces) e = copy(k + 1);
+      if (e == hipSuccess) e = hipEventSynchronize(buf.b[k & 1]->copied);
+      if (e != hipSuccess) return fail(TMPM_READBACK, std::string("device failure: ") + hipGetErrorString(e));
+      const float* data = buf.b[k & 1]->mem.data();
+      if (k == 0) {
+        const uint32_t* header = reinterpret_cast<const uint32_t*>(data);
+        std::memcpy(counters, header, 4 * CNT_COUNT);
+        tmpm_status st = check(header[CNT_COUNT], header[kReadbackHeader - 1] == mark);
+        if (st != TMPM_OK) return st;
+        data += kReadbackHeader;
+      }
+      widen_records(w, data, k * per, std::min(n - k * per, per), true, s->plastic);
     }
-    for (int q = 0; q < 9; ++q) {
-      w.C[9 * i + q] = C[q * n + slot];
-      w.F[9 * i + q] = F[q * n + slot];
-      finite = finite && std::isfinite(w.C[9 * i + q]) && std::isfinite(w.F[9 * i + q]);
-    }
-    if (s->plastic && is_plastic(w.material[i]))
-      for (int q = 0; q < 3; ++q) w.plastic[3 * i + q] = P[q * n + slot];
-    if (!finite) st[k] = TMPM_NON_FINITE_STATE;
   }
   return TMPM_OK;
 }
@@ -2303,8 +2382,11 @@ tmpm_status maybe_grow_topology(tmpm_session* s, const uint32_t* counters) {
 
 tmpm_status copy_particles_out(const HostWorld& w, tmpm_particles* out) {
   size_t n = std::min<size_t>(out->count, w.size());
+  // in parallel: the page faults of the caller's fresh arrays cost more than the copy
   auto put = [n](double* dst, const DVec& src, int k) {
-    if (dst) std::memcpy(dst, src.data(), sizeof(double) * k * n);
+    if (!dst) return;
+    parallel_for(n * k, [&](size_t b, size_t e) { std::memcpy(dst + b, src.data() + b, sizeof(double) * (e - b)); },
+                 1 << 17);
   };
   put(out->position, w.pos, 3);
   put(out->velocity, w.vel, 3);
@@ -2316,14 +2398,16 @@ tmpm_status copy_particles_out(const HostWorld& w, tmpm_particles* out) {
   put(out->radius, w.radius, 1);
   put(out->damping, w.damping, 1);
   put(out->plastic, w.plastic, 3);
-  for (size_t i = 0; i < n; ++i) {
-    if (out->group_id) out->group_id[i] = w.group_id[i];
-    if (out->transfer_color) out->transfer_color[i] = w.color[i];
-    if (out->enabled) out->enabled[i] = w.enabled[i];
-    if (out->fixed) out->fixed[i] = w.fixed[i];
-    if (out->chunk_id) out->chunk_id[i] = w.chunk[i];
-    if (out->material_index) out->material_index[i] = 0;
-  }
+  parallel_for(n, [&](size_t b, size_t e) {
+    for (size_t i = b; i < e; ++i) {
+      if (out->group_id) out->group_id[i] = w.group_id[i];
+      if (out->transfer_color) out->transfer_color[i] = w.color[i];
+      if (out->enabled) out->enabled[i] = w.enabled[i];
+      if (out->fixed) out->fixed[i] = w.fixed[i];
+      if (out->chunk_id) out->chunk_id[i] = w.chunk[i];
+      if (out->material_index) out->material_index[i] = 0;
+    }
+  }, 1 << 16);
   return TMPM_OK;
 }
 
@@ -3154,14 +3238,34 @@ tmpm_status tmpm_session_synchronize(tmpm_session* s) {
     const size_t ns = s->scenes.size();
     std::vector<uint32_t> scene_bits(ns, 0);
     uint32_t counters[CNT_COUNT] = {};
-    if (s->prepared) {
+    // Capacity and internal errors concern every scene: the session fails.  A
+    // single-scene session also fails on its scene's errors; a batch stops
+    // only the scenes concerned.
+    auto collect = [&]() -> tmpm_status {  // the device is done
+      collect_timers(s);
+      return s->audit_used ? collect_audit(s) : TMPM_OK;
+    };
+    auto take_counters = [&]() -> tmpm_status {  // the device is done, `counters` are read
+      const uint32_t global = s->batch ? (counters[CNT_ERROR] & (ERR_TOPOLOGY | ERR_INTERNAL)) : counters[CNT_ERROR];
+      tmpm_status st = status_from_error_bits(global);
+      if (st != TMPM_OK) return st;
+      s->last_pblocks = counters[CNT_PARTICLE_BLOCKS];
+      s->last_gblocks = counters[CNT_GRID_BLOCKS];
+      if (counters[CNT_REACT_SATURATED]) {
+        s->react_saturated += counters[CNT_REACT_SATURATED];
+        const uint32_t zero = 0;
+        if (hipMemcpy(s->counters.as<uint32_t>() + CNT_REACT_SATURATED, &zero, 4, hipMemcpyHostToDevice) != hipSuccess)
+          return fail(TMPM_READBACK, "counter reset failed");
+      }
+      return TMPM_OK;
+    };
+    if (s->prepared && s->batch) {
       hipError_t e = hipStreamSynchronize(s->stream);
       if (e != hipSuccess) {
         s->valid = false;
         return fail(TMPM_READBACK, std::string("device failure: ") + hipGetErrorString(e));
       }
-      collect_timers(s);
-      if (s->audit_used && collect_audit(s) != TMPM_OK) {
+      if (collect() != TMPM_OK) {
         s->valid = false;
         return TMPM_READBACK;
       }
@@ -3170,25 +3274,10 @@ tmpm_status tmpm_session_synchronize(tmpm_session* s) {
         s->valid = false;
         return fail(TMPM_READBACK, "counter readback failed");
       }
-      // Capacity and internal errors concern every scene: the session fails.
-      // A single-scene session also fails on its scene's errors; a batch stops
-      // only the scenes concerned.
-      const uint32_t global = s->batch ? (counters[CNT_ERROR] & (ERR_TOPOLOGY | ERR_INTERNAL)) : counters[CNT_ERROR];
-      tmpm_status st = status_from_error_bits(global);
+      tmpm_status st = take_counters();
       if (st != TMPM_OK) {
         s->valid = false;
         return st;
-      }
-      s->last_pblocks = counters[CNT_PARTICLE_BLOCKS];
-      s->last_gblocks = counters[CNT_GRID_BLOCKS];
-      if (counters[CNT_REACT_SATURATED]) {
-        s->react_saturated += counters[CNT_REACT_SATURATED];
-        const uint32_t zero = 0;
-        if (hipMemcpy(s->counters.as<uint32_t>() + CNT_REACT_SATURATED, &zero, 4, hipMemcpyHostToDevice) !=
-            hipSuccess) {
-          s->valid = false;
-          return fail(TMPM_READBACK, "counter reset failed");
-        }
       }
     }
     std::vector<char> commit(ns, 0);
@@ -3196,21 +3285,21 @@ tmpm_status tmpm_session_synchronize(tmpm_session* s) {
     bool coupling_read = false;
     if (!s->batch) {
       // eager: the world is read back at every synchronize
-      std::vector<HostWorld> updated;
-      std::vector<tmpm_status> scene_st;
-      st = read_back(s, updated, scene_st);
+      SceneState& scene = s->scenes[0];
+      st = read_back(s, counters, [&](uint32_t, bool not_finite) -> tmpm_status {
+        if (!s->prepared) return TMPM_OK;
+        tmpm_status c = collect();
+        if (c == TMPM_OK) c = take_counters();
+        if (c != TMPM_OK) return c;
+        return not_finite ? fail(TMPM_NON_FINITE_STATE, "MPM integration produced a non-finite state") : TMPM_OK;
+      });
       if (st != TMPM_OK) {
         s->valid = false;
         return st;
       }
-      if (scene_st[0] != TMPM_OK) {
-        s->valid = false;
-        return fail(scene_st[0], "MPM integration produced a non-finite state");
-      }
-      SceneState& scene = s->scenes[0];
       const uint64_t before = scene.world.substeps;
-      updated[0].substeps = before + steps < before ? UINT64_MAX : before + steps;
-      scene.set_world(updated[0]);
+      scene.world.substeps = before + steps < before ? UINT64_MAX : before + steps;
+      scene.stable = -1.0;
       commit[0] = 1;
     } else {
       // lazy: stopped scenes take their state of the previous synchronize from

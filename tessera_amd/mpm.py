@@ -441,12 +441,6 @@ class MpmParticle:
             enabled=self.enabled, fixed=self.fixed)
 
 
-def _column_major(m: np.ndarray) -> np.ndarray:
-    """(n, 3, 3) row-indexed view of a copy of `m` whose memory is column-major per matrix."""
-    buf = np.ascontiguousarray(np.transpose(m, (0, 2, 1)))
-    return buf.transpose(0, 2, 1)
-
-
 class ParticleArrays:
     """Structure-of-arrays particle storage in insertion order."""
 
@@ -458,8 +452,9 @@ class ParticleArrays:
         self.velocity = np.zeros((n, 3))
         # matrices are (n, 3, 3) views of column-major storage, the layout of
         # the C ABI (nalgebra order), so handing them to the library copies nothing
-        self.deformation = _column_major(np.tile(np.eye(3), (n, 1, 1)))
-        self.affine = _column_major(np.zeros((n, 3, 3)))
+        self.deformation = np.zeros((n, 3, 3)).transpose(0, 2, 1)
+        self.deformation[:, [0, 1, 2], [0, 1, 2]] = 1.0
+        self.affine = np.zeros((n, 3, 3)).transpose(0, 2, 1)
         self.force = np.zeros((n, 3))
         self.mass = np.zeros(n)
         self.rest_volume = np.zeros(n)
@@ -913,16 +908,17 @@ P2G_MODES = {"fp32": 0, "fixed64": 1}
 
 
 def _read_particle_arrays(n: int, read, lib) -> ParticleArrays:
-    """Reads n particles through `read(CParticles*)` into a ParticleArrays (row-major matrices)."""
-    out = ParticleArrays(n)
+    """Reads n particles through `read(CParticles*)` into a ParticleArrays (row-major matrices).
+    The library writes every element, so nothing is initialized first."""
+    out = ParticleArrays(0)
     flat = {
-        "position": np.zeros((n, 3)), "velocity": np.zeros((n, 3)), "deformation": np.zeros((n, 9)),
-        "affine": np.zeros((n, 9)), "force": np.zeros((n, 3)), "mass": np.zeros(n), "rest_volume": np.zeros(n),
-        "radius": np.zeros(n), "damping": np.zeros(n), "plastic": np.zeros((n, 3)),
+        "position": np.empty((n, 3)), "velocity": np.empty((n, 3)), "deformation": np.empty((n, 9)),
+        "affine": np.empty((n, 9)), "force": np.empty((n, 3)), "mass": np.empty(n), "rest_volume": np.empty(n),
+        "radius": np.empty(n), "damping": np.empty(n), "plastic": np.empty((n, 3)),
     }
     ints = {
-        "group_id": np.zeros(n, np.uint32), "transfer_color": np.zeros(n, np.uint16),
-        "enabled": np.zeros(n, np.uint8), "fixed": np.zeros(n, np.uint8), "chunk_id": np.zeros(n, np.uint64),
+        "group_id": np.empty(n, np.uint32), "transfer_color": np.empty(n, np.uint16),
+        "enabled": np.empty(n, np.uint8), "fixed": np.empty(n, np.uint8), "chunk_id": np.empty(n, np.uint64),
     }
     cp = CParticles()
     cp.count = n
@@ -946,8 +942,8 @@ def _read_particle_arrays(n: int, read, lib) -> ParticleArrays:
     out.plastic = flat["plastic"]
     out.group_id = ints["group_id"]
     out.transfer_color = ints["transfer_color"]
-    out.enabled = ints["enabled"].astype(bool)
-    out.fixed = ints["fixed"].astype(bool)
+    out.enabled = ints["enabled"].view(bool)
+    out.fixed = ints["fixed"].view(bool)
     out.chunk_id = ints["chunk_id"]
     return out
 

@@ -22,8 +22,8 @@ void launch_bin_update(const Parts& p, const Topo& t, const DevClass* c, const D
 void launch_p2g(const Parts& p, const Topo& t, const DevClass* c, const DevScene* sc, int fixed64, uint32_t blocks,
                 uint32_t threads, int copies, int plastic, hipStream_t s);
 // shapes != 0: some obstacle is a triangle prism or convex polyhedron
-void launch_grid_update(const Topo& t, const DevScene* sc, const DevObstacle* o, int fixed64, int react, int shapes,
-                        hipStream_t s);
+void launch_grid_update(const Topo& t, const DevScene* sc, const DevObstacle* o, uint32_t gblocks, int fixed64, int react,
+                        int shapes, hipStream_t s);
 // q: the reorder target (the whole state moved into block order), or empty
 void launch_g2p(const Parts& p, const Parts& q, const Topo& t, const DevClass* c, const DevScene* sc,
                 const DevObstacle* o, uint32_t blocks, uint32_t threads, int react, int shapes, int plastic,

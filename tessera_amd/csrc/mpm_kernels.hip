@@ -2104,7 +2104,7 @@ constexpr uint32_t kMoveOrderMax = 1024;
 constexpr uint32_t kMoveLevels = 128;  // particles per cell beyond which a block keeps its order
 
 template <int REACT, bool SHAPES, bool PLASTIC, bool MOVE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!SHAPES && !PLASTIC ? 5 : 1))) void k_g2p(
+__global__ __launch_bounds__(!SHAPES && !PLASTIC ? 512 : 256) __attribute__((amdgpu_waves_per_eu(!SHAPES && !PLASTIC ? 5 : 1))) void k_g2p(
     Parts p, Parts q, Topo t, const DevClass* __restrict__ classes, const DevScene* __restrict__ scenes,
     const DevObstacle* __restrict__ obstacles) {
   __shared__ float vt[3 * kTileNodes];
@@ -3049,23 +3049,26 @@ void launch_bin_update(const Parts& p, const Topo& t, const DevClass* c, const D
 }
 void launch_p2g(const Parts& p, const Topo& t, const DevClass* c, const DevScene* sc, int fixed64, uint32_t blocks,
                 uint32_t threads, int copies, int plastic, hipStream_t s) {
-  // sessions with plastic materials run the default shape (64 threads, 2 tile copies)
-  if (plastic) {
-    if (fixed64) hipLaunchKernelGGL((k_p2g<1, 64, 2, true>), dim3(blocks), dim3(64), 0, s, p, t, c, sc);
-    else hipLaunchKernelGGL((k_p2g<0, 64, 2, true>), dim3(blocks), dim3(64), 0, s, p, t, c, sc);
-    return;
-  }
-  // threads per workgroup: 64 or 128 (anything else runs 128); LDS tile copies: 1 or 2
-#define TMPM_P2G(F, T, K) hipLaunchKernelGGL((k_p2g<F, T, K, false>), dim3(blocks), dim3(T), 0, s, p, t, c, sc)
-#define TMPM_P2G_T(F, K)                  \
-  do {                                    \
-    if (threads == 64) TMPM_P2G(F, 64, K); \
-    else TMPM_P2G(F, 128, K);              \
+  // threads per workgroup: 64 or 128 with 1 or 2 LDS tile copies, 256 or 512
+  // with one (anything else runs 128).  Plastic sessions run 128 instead of 64
+  // and one copy: sand, 2,744 blocks of 292
+  // and 8,788 of 114: 46.9 and 55.1 us; with 64 threads and two copies 51.7 and
+  // 65.4.
+#define TMPM_P2G(F, T, K, P) hipLaunchKernelGGL((k_p2g<F, T, K, P>), dim3(blocks), dim3(T), 0, s, p, t, c, sc)
+#define TMPM_P2G_T(F, P)                                   \
+  do {                                                     \
+    if (threads == 512) TMPM_P2G(F, 512, 1, P);            \
+    else if (threads == 256) TMPM_P2G(F, 256, 1, P);       \
+    else if (P) TMPM_P2G(F, 128, 1, P);                    \
+    else if (threads == 64 && copies == 2) TMPM_P2G(F, 64, 2, false); \
+    else if (threads == 64) TMPM_P2G(F, 64, 1, false);     \
+    else if (copies == 2) TMPM_P2G(F, 128, 2, false);      \
+    else TMPM_P2G(F, 128, 1, false);                       \
   } while (0)
-  if (fixed64) {
-    if (copies == 2) TMPM_P2G_T(1, 2); else TMPM_P2G_T(1, 1);
+  if (plastic) {
+    if (fixed64) TMPM_P2G_T(1, true); else TMPM_P2G_T(0, true);
   } else {
-    if (copies == 2) TMPM_P2G_T(0, 2); else TMPM_P2G_T(0, 1);
+    if (fixed64) TMPM_P2G_T(1, false); else TMPM_P2G_T(0, false);
   }
 #undef TMPM_P2G_T
 #undef TMPM_P2G
@@ -3081,9 +3084,9 @@ static void grid_update_variant(const Topo& t, const DevScene* sc, const DevObst
     else hipLaunchKernelGGL((k_grid_update<0, 0, SHAPES>), dim3(blocks), dim3(256), 0, s, t, sc, o);
   }
 }
-void launch_grid_update(const Topo& t, const DevScene* sc, const DevObstacle* o, int fixed64, int react, int shapes,
-                        hipStream_t s) {
-  uint32_t blocks = grid_for(t.grid_cap, 4, 16384);
+void launch_grid_update(const Topo& t, const DevScene* sc, const DevObstacle* o, uint32_t gblocks, int fixed64, int react,
+                        int shapes, hipStream_t s) {
+  uint32_t blocks = grid_for(gblocks, 4, 16384);
   if (shapes) grid_update_variant<true>(t, sc, o, fixed64, react, blocks, s);
   else grid_update_variant<false>(t, sc, o, fixed64, react, blocks, s);
 }

@@ -1795,7 +1795,7 @@ struct SubstepPlan {
   DevRigid* rigid;
   const DevMapping* maps;
   const uint32_t* body_scene;
-  uint32_t obstacle_total, body_total, p2g_blocks, p2g_threads, g2p_threads;
+  uint32_t obstacle_total, body_total, pblocks, gblocks, p2g_threads, g2p_threads;
   int32_t react, fixed64, shapes, plastic, cpic, copies;
   double* audit;  // FP64 audit record set of this substep, or null
   uint8_t reorder, clear_table, rigid_sync, rigid_apply;
@@ -1814,16 +1814,59 @@ struct SubstepPlan {
 //     21,187 blocks of 252: 390 us at 128, 400 at 64 and 256; serving
 //     batches of 3,123 blocks of 313 and 8,916 of 345: 112 -> 81 and
 //     326 -> 284 us from 64 to 256 threads.
+//     With plastic materials G2P holds 2 wavefronts per SIMD, and idle ones of
+//     a block's workgroup keep others out: from a block per CU on, no wider
+//     than the mean block has particles, and no wider than 128 from four
+//     blocks per CU on (1,000 blocks of 80 sand particles: 35.5 us at 256,
+//     18.5 at 128, 25.9 at 64; 576 of 260: 36.4, 45.2, 67.4; 2,744 of 292:
+//     117, 112, 129).
 //   P2G: 128 threads below kFillBlocks or from 192 particles per block, else
 //     64 (1M particles: 76 vs 86 us at 128; the batches above: 1-4% faster
 //     at 128); one tile copy.  The reorder deals each block's particles
 //     round-robin by cell, so a wavefront's lanes rarely share a cell, and a
 //     second copy's LDS costs more workgroups per CU than the same-address
 //     atomics it separates (1M particles: 61 vs 66 us).
-constexpr uint32_t kFillBlocks = 8192;  // 32 waves per CU of MI355X's 256
+int floor_log2(uint64_t v) { return v ? 63 - __builtin_clzll(v) : -1; }
+
+constexpr uint32_t kCus = 256;               // MI355X
+constexpr uint32_t kFillBlocks = 32 * kCus;  // 32 waves per CU
 
 uint32_t particles_per_block(const tmpm_session* s) {
   return s->last_pblocks ? (uint32_t)(s->n / s->last_pblocks) : 0u;
+}
+
+// The launch of a shape's widest workgroups (P2G's 128 threads, G2P's 256) goes
+// wider yet while the chip has room for all blocks at once: 16 wavefronts per
+// CU of P2G and 20 of the plain G2P are resident, so two workgroups of 512
+// threads each, or four of 256.  A few blocks are then as fast as their longest
+// chain: the passes over the particles, P2G's flush and the tile loads, all
+// shorter the wider the workgroup.  Measured (us at 64 / 128 / 256 / 512):
+//   P2G   77 blocks of 106: 20.4 / 14.0 / 11.0 / 9.8;  342 of 173: 27.6 /
+//         18.5 / 13.3 / 12.1;  503 of 239: 29 / 19.9 / 13.4 / 12.5;  716 of 70:
+//         16.3 / 13.9 / 11.2 / 14.4;  900 of 278: 33 / 24.4 / 19.9 / 20.6;
+//         1,243 of 80: 18.4 / 15.5 / 15.6 / 19.4;  2,386 of 84: 24.5 / 22.7 /
+//         22.6 / 31.6.
+//   G2P   77 of 106: 25.7 / 18.0 / 13.8 / 9.6;  342 of 173: 35.1 / 22.9 / 14.7 /
+//         11.8;  503 of 239: 38 / 25.3 / 16.2 / 13.2;  716 of 70: 18.5 / 14.2 /
+//         10.6 / 15.4;  900 of 278: 43.8 / 29.7 / 20.3 / 22.6.
+uint32_t widened_p2g(const tmpm_session* s, uint32_t threads, int copies) {
+  const uint32_t b = s->last_pblocks;
+  if (threads != 128 || copies != 1 || b > 4 * kCus) return threads;
+  return b <= 2 * kCus ? 512u : 256u;
+}
+uint32_t widened_g2p(const tmpm_session* s, uint32_t threads) {
+  return threads == 256 && !s->plastic && !s->shapes && s->last_pblocks <= 2 * kCus ? 512u : threads;
+}
+
+// Workgroups of a launch that takes one block each (every kernel strides over
+// the rest): an eighth more than the last synchronized count, in steps of an
+// eighth, so that a captured plan holds for a while.  Launched for the whole
+// capacity, four times the blocks at the start, three of four workgroups
+// found no block.
+uint32_t launch_blocks(uint32_t last, uint32_t most) {
+  const uint64_t want = last + last / 8 + 64;
+  const uint32_t step = 1u << (floor_log2(want) - 3);
+  return (uint32_t)std::min<uint64_t>(most, (want + step - 1) / step * step);
 }
 
 // Autotuner cache.  Tuned launch shapes are kept per workload bucket: device,
@@ -1906,8 +1949,6 @@ TuneCache& tune_cache() {
   return c;
 }
 
-int floor_log2(uint64_t v) { return v ? 63 - __builtin_clzll(v) : -1; }
-
 TuneKey tune_key(const tmpm_session* s) {
   TuneKey k;
   k.device = s->ctx ? s->ctx->device : 0;
@@ -1928,7 +1969,9 @@ uint32_t effective_g2p_threads(const tmpm_session* s) {
   const uint32_t b = s->last_pblocks, ppb = particles_per_block(s);
   const uint32_t by_blocks = b >= kFillBlocks ? 64u : b >= kFillBlocks / 2 ? 128u : 256u;
   const uint32_t by_density = ppb >= 288 ? 256u : ppb >= 192 ? 128u : 64u;
-  return std::max(by_blocks, by_density);
+  const uint32_t threads = std::max(by_blocks, by_density);
+  if (!s->plastic || b <= kCus || ppb == 0) return threads;
+  return std::min(threads, ppb <= 64 ? 64u : ppb <= 128 || b > 4 * kCus ? 128u : 256u);
 }
 
 void effective_p2g_shape(const tmpm_session* s, uint32_t& threads, int& copies) {
@@ -1944,7 +1987,7 @@ void effective_p2g_shape(const tmpm_session* s, uint32_t& threads, int& copies) 
     return;
   }
   const uint32_t b = s->last_pblocks;
-  threads = b < kFillBlocks || particles_per_block(s) >= 192 ? 128u : 64u;
+  threads = b < kFillBlocks || particles_per_block(s) >= 192 || s->plastic ? 128u : 64u;
   copies = 1;
 }
 
@@ -1987,9 +2030,11 @@ SubstepPlan plan_substep(tmpm_session* s, bool apply_force) {
   pl.body_scene = s->body_scene.as<uint32_t>();
   pl.obstacle_total = s->obstacle_total;
   pl.body_total = s->body_total;
-  pl.p2g_blocks = s->p2g_blocks;
+  pl.pblocks = launch_blocks(s->last_pblocks, s->p2g_blocks);
+  pl.gblocks = launch_blocks(s->last_gblocks, s->topo.grid_cap);
   effective_p2g_shape(s, pl.p2g_threads, pl.copies);
-  pl.g2p_threads = effective_g2p_threads(s);
+  pl.p2g_threads = widened_p2g(s, pl.p2g_threads, pl.copies);
+  pl.g2p_threads = widened_g2p(s, effective_g2p_threads(s));
   pl.react = s->react_active() && s->obstacle_total > 0 ? 1 : 0;
   pl.fixed64 = s->fixed64 ? 1 : 0;
   pl.shapes = s->shapes;
@@ -2032,15 +2077,15 @@ hipError_t launch_plan(tmpm_session* s, const SubstepPlan& pl) {
     if ((e = timed(s, "k_bin_scatter", [&] { launch_bin_scatter(p, t, st); })) != hipSuccess) return e;
   }
   if ((e = timed(s, pl.fixed64 ? "k_p2g_fixed64" : "k_p2g", [&] {
-         launch_p2g(p, t, pl.c, pl.sc, pl.fixed64, pl.p2g_blocks, pl.p2g_threads, pl.copies, pl.plastic, st);
+         launch_p2g(p, t, pl.c, pl.sc, pl.fixed64, pl.pblocks, pl.p2g_threads, pl.copies, pl.plastic, st);
        })) != hipSuccess)
     return e;
   if ((e = timed(s, "k_grid_update",
-                 [&] { launch_grid_update(t, pl.sc, pl.ob, pl.fixed64, pl.react, pl.shapes, st); })) != hipSuccess)
+                 [&] { launch_grid_update(t, pl.sc, pl.ob, pl.gblocks, pl.fixed64, pl.react, pl.shapes, st); })) != hipSuccess)
     return e;
   if ((e = timed(s, "k_g2p", [&] {
          // on a reorder substep G2P also moves the state into block order in q
-         launch_g2p(p, pl.q, t, pl.c, pl.sc, pl.ob, pl.p2g_blocks, pl.g2p_threads, pl.react, pl.shapes, pl.plastic,
+         launch_g2p(p, pl.q, t, pl.c, pl.sc, pl.ob, pl.pblocks, pl.g2p_threads, pl.react, pl.shapes, pl.plastic,
                     st);
        })) != hipSuccess)
     return e;

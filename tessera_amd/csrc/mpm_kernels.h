@@ -44,9 +44,10 @@ void launch_gather_state(const Parts& p, const DevClass* c, const Topo& t, uint3
                          hipStream_t s);
 void launch_copy(const float4* src, float4* dst, size_t n, hipStream_t s);
 // flags[c] = 1 for lattice candidate c (x-major, then y, then z) inside the closed mesh
+uint32_t mesh_parts(uint64_t count, uint64_t ntri);  // of launch_mesh_inside; `part` holds 8 bytes per candidate and part
 void launch_mesh_inside(const double* verts, const uint32_t* tris, uint64_t ntri, const double lower[3],
-                        const double upper[3], double spacing, const uint64_t counts[3], uint8_t* flags,
-                        hipStream_t s);
+                        const double upper[3], double spacing, const uint64_t counts[3], uint8_t* flags, double* part,
+                        uint32_t parts, hipStream_t s);
 // *bad = 1 unless every directed edge of the triangles occurs exactly once
 // and its reverse exactly once (the caller zeroes *bad)
 void launch_mesh_edges(const uint32_t* tris, uint64_t ntri, uint32_t* bad, hipStream_t s);

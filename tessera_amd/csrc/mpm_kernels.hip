@@ -2864,8 +2864,9 @@ __global__ __launch_bounds__(256) void k_live_count(Topo t) {
 // candidate lies on the surface, or the mesh's scale over- or underflows), the
 // candidate is left to k_mesh_inside, one thread per candidate that sums the
 // angles in the reference's order.
-// Bound by f64 issue (75 f64 operations per pair).  1,280 triangles and 18,400
-// candidates: 137 us, and 4 us for k_mesh_inside over the undecided ones; 704 us
+// Bound by f64 issue (75 f64 operations per pair, ~50 us of it on all CUs).
+// 1,280 triangles and 18,400 candidates: 84 us, and 4 us for k_mesh_inside over
+// the undecided ones; 137 us with each group's triangles in one workgroup; 704 us
 // with an atan2 per pair on one thread per candidate (72 workgroups).
 // ---------------------------------------------------------------------------
 constexpr uint8_t kMeshUndecided = 2;
@@ -2876,16 +2877,23 @@ __device__ __forceinline__ double mesh_root(double x) {
   return __builtin_fma(0.5 * y, __builtin_fma(-r, r, x), r);
 }
 
+// From the whole sum (NaN: undecided): a turn and more, none, or in between.
+__device__ __forceinline__ uint8_t mesh_decide(double angle) {
+  const double a = fabs(angle);
+  return !(fabs(a - 3.141592653589793) > 1.0) ? kMeshUndecided : a > 3.141592653589793 ? 1 : 0;
+}
+
 __global__ __launch_bounds__(1024) void k_mesh_winding(const double* __restrict__ verts,
                                                        const uint32_t* __restrict__ tris, uint64_t ntri, double lx,
                                                        double ly, double lz, double spacing, uint64_t cy, uint64_t cz,
                                                        double ux, double uy, double uz, uint64_t count,
-                                                       uint8_t* flags) {
+                                                       uint8_t* flags, double* __restrict__ part) {
   __shared__ double s_angle[16][64];
   __shared__ uint32_t s_near[16][64];
   const uint32_t lane = threadIdx.x & 63, waves = blockDim.x >> 6;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint64_t t0 = ntri * wave / waves, t1 = ntri * (wave + 1) / waves;
+  const uint64_t share = (uint64_t)blockIdx.y * waves + wave, shares = (uint64_t)gridDim.y * waves;
+  const uint64_t t0 = ntri * share / shares, t1 = ntri * (share + 1) / shares;
   for (uint64_t c0 = (uint64_t)blockIdx.x * 64; c0 < count; c0 += (uint64_t)gridDim.x * 64) {
     const uint64_t c = c0 + lane;
     const uint64_t x = c / (cy * cz), y = (c / cz) % cy, z = c % cz;
@@ -2929,22 +2937,28 @@ __global__ __launch_bounds__(1024) void k_mesh_winding(const double* __restrict_
         angle += s_angle[w][lane];
         undecided |= s_near[w][lane];
       }
-      const double a = fabs(angle);
-      const bool out = px >= ux || py >= uy || pz >= uz;
-      flags[c] = out ? 0 : undecided || !(fabs(a - 3.141592653589793) > 1.0) ? kMeshUndecided : a > 3.141592653589793;
+      if (undecided) angle = __builtin_nan("");
+      if (gridDim.y > 1) part[blockIdx.y * count + c] = angle;
+      else flags[c] = px >= ux || py >= uy || pz >= uz ? 0 : mesh_decide(angle);
     }
     __syncthreads();
   }
 }
 
-// The candidates that k_mesh_winding left undecided.
+// Adds up the parts of k_mesh_winding, and decides the candidates that it left
+// undecided.
 __global__ __launch_bounds__(256) void k_mesh_inside(const double* __restrict__ verts,
                                                      const uint32_t* __restrict__ tris, uint64_t ntri,
                                                      double lx, double ly, double lz, double spacing, uint64_t cy,
                                                      uint64_t cz, double ux, double uy, double uz, uint64_t count,
-                                                     uint8_t* flags) {
+                                                     uint8_t* flags, const double* __restrict__ part,
+                                                     uint32_t parts) {
   for (uint64_t c = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; c < count; c += (uint64_t)gridDim.x * blockDim.x) {
-    if (flags[c] != kMeshUndecided) continue;
+    if (parts > 1) {
+      double angle = 0.0;
+      for (uint32_t q = 0; q < parts; ++q) angle += part[q * count + c];
+      flags[c] = mesh_decide(angle);
+    }
     const uint64_t x = c / (cy * cz), y = (c / cz) % cy, z = c % cz;
     const double px = lx + ((double)x + 0.5) * spacing;
     const double py = ly + ((double)y + 0.5) * spacing;
@@ -2953,6 +2967,7 @@ __global__ __launch_bounds__(256) void k_mesh_inside(const double* __restrict__ 
       flags[c] = 0;
       continue;
     }
+    if (flags[c] != kMeshUndecided) continue;
     double angle = 0.0;
     for (uint64_t t = 0; t < ntri; ++t) {
       double v[3][3];
@@ -3190,19 +3205,31 @@ void launch_live_nodes(const Parts& p, const Topo& t, const DevClass* c, const D
   hipLaunchKernelGGL(k_live_count, dim3(grid_for(2ull * t.grid_cap, 256, 4096)), dim3(256), 0, s, t);
 }
 
+// Where the 64-candidate groups are few, their triangles are also split over
+// workgroups of kMeshPartWaves wavefronts, as many parts as give each CU 8 of
+// them: 286 groups were 1 workgroup of 16 wavefronts on most CUs and 2 on the
+// others, which took twice as long (137 us against 84).  At least 8 triangles per wavefront.  The
+// parts' sums (8 bytes per candidate and part) go to `part`.
+constexpr uint32_t kMeshPartWaves = 4;
+uint32_t mesh_parts(uint64_t count, uint64_t ntri) {
+  const uint64_t groups = (count + 63) / 64;
+  const uint64_t want = groups ? (2048 + groups - 1) / groups : 1, most = ntri / (8 * kMeshPartWaves);
+  return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(std::min(want, most), 64));
+}
 void launch_mesh_inside(const double* verts, const uint32_t* tris, uint64_t ntri, const double lower[3],
-                        const double upper[3], double spacing, const uint64_t counts[3], uint8_t* flags,
-                        hipStream_t s) {
+                        const double upper[3], double spacing, const uint64_t counts[3], uint8_t* flags, double* part,
+                        uint32_t parts, hipStream_t s) {
   const uint64_t count = counts[0] * counts[1] * counts[2];
-  // Wavefronts per workgroup, which share its 64 candidates' triangles: 16 until
-  // that makes 64 waves per SIMD, and at least 8 triangles each.
-  uint32_t waves = 16;
-  while (waves > 1 && (waves * ((count + 63) / 64) > 65536 || ntri < 8ull * waves)) waves /= 2;
-  hipLaunchKernelGGL(k_mesh_winding, dim3(grid_for(count, 64, 1u << 20)), dim3(64 * waves), 0, s, verts, tris, ntri,
-                     lower[0], lower[1], lower[2], spacing, counts[1], counts[2], upper[0], upper[1], upper[2], count,
-                     flags);
+  // Wavefronts per workgroup, which share its 64 candidates' triangles: in one
+  // part 16 until that makes 64 waves per SIMD, and at least 8 triangles each.
+  uint32_t waves = parts > 1 ? kMeshPartWaves : 16;
+  while (parts == 1 && waves > 1 && (waves * ((count + 63) / 64) > 65536 || ntri < 8ull * waves)) waves /= 2;
+  hipLaunchKernelGGL(k_mesh_winding, dim3(grid_for(count, 64, 1u << 20), parts), dim3(64 * waves), 0, s, verts, tris,
+                     ntri, lower[0], lower[1], lower[2], spacing, counts[1], counts[2], upper[0], upper[1], upper[2],
+                     count, flags, part);
   hipLaunchKernelGGL(k_mesh_inside, dim3(grid_for(count, 256, 65536)), dim3(256), 0, s, verts, tris, ntri, lower[0],
-                     lower[1], lower[2], spacing, counts[1], counts[2], upper[0], upper[1], upper[2], count, flags);
+                     lower[1], lower[2], spacing, counts[1], counts[2], upper[0], upper[1], upper[2], count, flags,
+                     part, parts);
 }
 void launch_mesh_edges(const uint32_t* tris, uint64_t ntri, uint32_t* bad, hipStream_t s) {
   hipLaunchKernelGGL(k_mesh_edges, dim3(grid_for(3 * ntri, 256, 4096)), dim3(256), 0, s, tris, ntri, bad);

@@ -2549,6 +2549,12 @@ NoAllocScratch& noalloc_scratch(int device) {
   return table[device & 255];
 }
 
+// As many of the sampler's parts as the scratch memory holds from `offset` on.
+uint32_t mesh_parts_within(uint32_t parts, uint64_t candidates, uint64_t offset) {
+  while (parts > 1 && (offset > kScratchBytes || 8ull * candidates * parts > kScratchBytes - offset)) parts /= 2;
+  return parts;
+}
+
 // Looks up this device's address of `scratch`; the device must be current.
 tmpm_status setup_scratch(int device) {
   void* ptr = nullptr;
@@ -4311,14 +4317,17 @@ tmpm_status tmpm_sample_closed_mesh_volume(tmpm_context* ctx, const double* vert
     // enough.  The host tests the edges meanwhile.
     if (hipSetDevice(ctx->device) != hipSuccess) return fail(TMPM_NO_DEVICE, "cannot select device");
     const uint64_t off_t = 24ull * vertex_count, off_f = off_t + 12ull * triangle_count;
+    const uint64_t off_p = (off_f + lat.candidates + 255) & ~uint64_t(255);
+    uint32_t parts = mesh_parts(lat.candidates, triangle_count);
     NoAllocScratch& ns = noalloc_scratch(ctx->device);
     std::unique_lock<std::mutex> lock(ns.mu, std::defer_lock);
     DevBuf own;
     char* base = nullptr;
     if (off_f + lat.candidates <= kScratchBytes && ns.ptr && lock.try_lock()) {
       base = static_cast<char*>(ns.ptr);
+      parts = mesh_parts_within(parts, lat.candidates, off_p);
     } else {
-      HIP_TRY(own.alloc(off_f + lat.candidates));
+      HIP_TRY(own.alloc(off_p + (parts > 1 ? 8ull * lat.candidates * parts : 0)));
       base = static_cast<char*>(own.ptr);
     }
     std::vector<char> mesh(off_f);
@@ -4335,7 +4344,7 @@ tmpm_status tmpm_sample_closed_mesh_volume(tmpm_context* ctx, const double* vert
     HIP_TRY(hipMemcpyAsync(base, mesh.data(), off_f, hipMemcpyHostToDevice, stream.s));
     launch_mesh_inside(reinterpret_cast<const double*>(base), reinterpret_cast<const uint32_t*>(base + off_t),
                        triangle_count, lat.lower, lat.upper, spacing, lat.counts, reinterpret_cast<uint8_t*>(base + off_f),
-                       stream.s);
+                       reinterpret_cast<double*>(base + off_p), parts, stream.s);
     hipError_t e = hipGetLastError();
     bool closed = false, threw = false;
     try {
@@ -4401,7 +4410,10 @@ tmpm_status tmpm_sample_closed_mesh_volume_noalloc(tmpm_context* ctx, const doub
     if ((st = mesh_lattice(vertices, vertex_count, spacing, max_candidates, lat)) != TMPM_OK) return st;
     if (lat.candidates > kScratchBytes - off_f)
       return fail(TMPM_CAPACITY, "candidate lattice exceeds the allocation-free sampler's scratch memory");
-    launch_mesh_inside(dv, dt, triangle_count, lat.lower, lat.upper, spacing, lat.counts, df, nullptr);
+    const uint64_t off_p = align(off_f + lat.candidates);
+    launch_mesh_inside(dv, dt, triangle_count, lat.lower, lat.upper, spacing, lat.counts, df,
+                       reinterpret_cast<double*>(base + off_p),
+                       mesh_parts_within(mesh_parts(lat.candidates, triangle_count), lat.candidates, off_p), nullptr);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return fail(TMPM_READBACK, std::string("mesh sampling kernel failed: ") + hipGetErrorString(e));

@@ -34,6 +34,9 @@ void launch_rigid_apply(const Topo& t, const DevScene* sc, DevRigid* bodies, con
                         const DevObstacle* o, const uint32_t* body_scene, uint32_t count, hipStream_t s);
 void launch_rigid_step(const Topo& t, const DevScene* sc, DevRigid* bodies, const DevMapping* maps, DevObstacle* o,
                        const uint32_t* body_scene, uint32_t body_total, int sync, hipStream_t s);
+void launch_update_rigid(const Parts& p, const Topo& t, const DevClass* c, const DevScene* sc, DevRigid* bodies,
+                         const DevMapping* maps, DevObstacle* o, const uint32_t* body_scene, uint32_t body_total,
+                         hipStream_t s);
 void launch_snapshot(const Parts& p, float4* out, hipStream_t s);
 void launch_snapshot_disabled(const float4* rec, uint32_t count, float4* out, hipStream_t s);
 void launch_retire(const Parts& p, uint32_t first, uint32_t count, hipStream_t s);

@@ -660,6 +660,7 @@ struct tmpm_session {
     bin_stage, bin_nstage, bin_claims, bin_nclaims, bin_csum, bmask, pmask, stray;
   DevBuf list_meta[2], list_idx[2];  // block lists, read and written in turn
   bool lists_valid = false;  // the last substep left the next one's block lists and the block table
+  bool rigid_pending = false;  // within a submission: the next substep runs the last one's rigid step
   int list_read = 0;         // the set the next listed substep reads
   Topo topo{};
   uint32_t p2g_blocks = 4096, threads_pblock = 64, p2g_threads = 64;
@@ -1798,7 +1799,7 @@ struct SubstepPlan {
   uint32_t obstacle_total, body_total, pblocks, gblocks, p2g_threads, g2p_threads;
   int32_t react, fixed64, shapes, plastic, cpic, copies;
   double* audit;  // FP64 audit record set of this substep, or null
-  uint8_t reorder, clear_table, rigid_sync, rigid_apply, rigid_step, rigid_next;
+  uint8_t reorder, clear_table, rigid_sync, rigid_apply, rigid_step, rigid_next, rigid_before;
 };
 
 // Default launch shapes, from the particle-block count of the last
@@ -2051,9 +2052,13 @@ SubstepPlan plan_substep(tmpm_session* s, bool apply_force, bool first, bool mor
   // leaves the poses it ran with: synchronize reads those.
   const bool coupled = s->body_total > 0 && s->obstacle_total > 0;
   pl.rigid_apply = pl.react && s->body_total > 0;
-  pl.rigid_step = pl.rigid_apply && std::max(s->obstacle_total, s->body_total) <= kRigidStepMost;
-  pl.rigid_next = pl.rigid_step && more;
-  pl.rigid_sync = coupled && (first || (pl.rigid_apply && !pl.rigid_step));
+  const bool one_step = pl.rigid_apply && std::max(s->obstacle_total, s->body_total) <= kRigidStepMost;
+  pl.rigid_sync = coupled && (first || (pl.rigid_apply && !one_step));
+  // The listed substep that follows a `build` takes the rigid step into its
+  // launch of k_bin_update (k_update_rigid).
+  pl.rigid_before = listed && s->rigid_pending;
+  pl.rigid_next = one_step && more;
+  pl.rigid_step = one_step && !(more && build);
   pl.audit = s->audit_on ? s->audit_next : nullptr;
   return pl;
 }
@@ -2073,7 +2078,12 @@ hipError_t launch_plan(tmpm_session* s, const SubstepPlan& pl) {
   if (pl.cpic &&
       (e = timed(s, "k_cpic_mask", [&] { launch_cpic_mask(p, t, pl.c, pl.sc_plain, pl.ob, st); })) != hipSuccess)
     return e;
-  if (t.listed) {
+  if (pl.rigid_before) {
+    if ((e = timed(s, "k_update_rigid", [&] {
+           launch_update_rigid(p, t, pl.c, pl.sc_plain, pl.rigid, pl.maps, pl.ob, pl.body_scene, pl.body_total, st);
+         })) != hipSuccess)
+      return e;
+  } else if (t.listed) {
     if ((e = timed(s, "k_bin_update", [&] { launch_bin_update(p, t, pl.c, pl.sc_plain, st); })) != hipSuccess)
       return e;
   } else {
@@ -2100,15 +2110,16 @@ hipError_t launch_plan(tmpm_session* s, const SubstepPlan& pl) {
                     st);
        })) != hipSuccess)
     return e;
+  const bool three = !pl.rigid_step && !pl.rigid_next;
   if (pl.rigid_step) {
     if ((e = timed(s, "k_rigid_step", [&] {
            launch_rigid_step(t, pl.sc, pl.rigid, pl.maps, pl.ob, pl.body_scene, pl.body_total,
                              pl.rigid_next, st);
          })) != hipSuccess)
       return e;
-  } else if (pl.react && (e = timed(s, "k_react_finalize", [&] { launch_react_finalize(t, pl.ob, st); })) != hipSuccess)
+  } else if (three && pl.react && (e = timed(s, "k_react_finalize", [&] { launch_react_finalize(t, pl.ob, st); })) != hipSuccess)
     return e;
-  if (pl.rigid_apply && !pl.rigid_step && (e = timed(s, "k_rigid_apply", [&] {
+  if (three && pl.rigid_apply && (e = timed(s, "k_rigid_apply", [&] {
                            launch_rigid_apply(t, pl.sc, pl.rigid, pl.maps, pl.ob, pl.body_scene, pl.body_total, st);
                          })) != hipSuccess)
     return e;
@@ -2172,6 +2183,7 @@ hipError_t enqueue_substep(tmpm_session* s, bool apply_force, bool first, bool m
   const hipError_t e = s->use_graphs && !s->timing && !pl.audit ? launch_graph(s, pl) : launch_plan(s, pl);
   if (e != hipSuccess) return e;
   s->lists_valid = pl.t.build != 0;
+  s->rigid_pending = pl.rigid_next && !pl.rigid_step;
   s->list_read = pl.t.listed ? 1 - s->list_read : 1;
   s->table_dirty = pl.t.build != 0;  // otherwise G2P cleared the block table
   if (pl.reorder) {

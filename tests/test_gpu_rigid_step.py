@@ -64,3 +64,21 @@ def test_more_obstacles_than_one_workgroup_takes(transfers):
         same(alone.rigid_bodies()[0], batch.rigid_bodies(k)[0], alone.obstacles(), batch.obstacles(k))
         assert np.array_equal(alone.read_particles().position, batch.read_particles(k).position)
         alone.close()
+
+
+def test_rigid_step_of_a_submission_over_reorders(transfers):
+    # the rigid step rides on the next substep's list update except before a reorder and at the end
+    w, bodies, maps = crowded(1, 3)
+    dt = min(5.0e-5, 0.5 * w.stable_timestep())
+    runs = []
+    for parts in ((40,), (1,) * 40, (15, 2, 16, 7)):
+        s = HipMpmResidentSession(transfers, w, dt, "fixed64")
+        s.set_rigid_bodies(bodies, maps, gravity=G, integrate=True)
+        for k in parts:
+            s.submit_steps(k)
+        s.synchronize()
+        runs.append((s.rigid_bodies()[0], s.obstacles(), s.reactions(), s.read_particles().position))
+        s.close()
+    for body, obstacles, reactions, position in runs[1:]:
+        same(runs[0][0], body, runs[0][1], obstacles)
+        assert np.array_equal(runs[0][2], reactions) and np.array_equal(runs[0][3], position)

@@ -245,6 +245,9 @@ struct Topo {
   // and the block whose entries for it are taken (its place beyond them is in
   // pslot), or kInvalid where its block is to be looked up, and maybe made.
   uint2* stray;
+  // pinned host memory (or null): particle and grid blocks of the last full
+  // binning, which the host's next launch shapes follow without waiting
+  uint32_t* seen;
 };
 
 }  // namespace tmpm

@@ -663,6 +663,8 @@ __device__ __forceinline__ void pblock_finalize(const Topo& t) {
 constexpr int kScatterK = 4;
 __global__ __launch_bounds__(256) void k_bin_scatter(Parts p, Topo t) {
   pblock_finalize(t);
+  if (t.seen && blockIdx.x == 0 && threadIdx.x < 2)
+    t.seen[threadIdx.x] = t.counters[threadIdx.x ? CNT_GRID_BLOCKS : CNT_PARTICLE_BLOCKS];
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x; i0 < p.n; i0 += kScatterK * stride) {
     uint32_t b[kScatterK], r[kScatterK], st[kScatterK];

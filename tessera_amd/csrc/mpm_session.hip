@@ -633,6 +633,18 @@ struct tmpm_session {
   std::vector<HostWorld> spare_worlds;  // emptied worlds of retired scenes, reused
   uint32_t force_cap = 0;
   uint32_t last_pblocks = 0, last_gblocks = 0;  // block counts of the last synchronized substep
+  uint32_t* seen = nullptr;                     // Topo::seen: those of the last full binning, 0 for none since
+  ~tmpm_session() {
+    if (seen) (void)hipHostFree(seen);
+  }
+  void forget_seen() {
+    if (seen) seen[0] = seen[1] = 0;
+  }
+  // Blocks to launch for: a session may run for long without a synchronize, and
+  // a spreading scene leaves the count it began with (sand, 79,507 particles from
+  // 1,000 blocks, a frame of 10 substeps: 280 us by the first count, 245 by these).
+  uint32_t pblocks_now() const { return std::max(last_pblocks, seen ? ((const volatile uint32_t*)seen)[0] : 0u); }
+  uint32_t gblocks_now() const { return std::max(last_gblocks, seen ? ((const volatile uint32_t*)seen)[1] : 0u); }
   uint32_t topo_cap = 0;   // particle capacity the topology's per-particle arrays were sized for
   std::map<ClassKey, uint32_t> class_ids;
   DevBuf force;            // float4 per particle, insertion order
@@ -1199,6 +1211,13 @@ tmpm_status alloc_topology(tmpm_session* s, uint32_t pblock_cap, uint32_t grid_c
   t.grid_rev = s->grid_rev.as<uint32_t>();
   t.grid_vel = s->grid_vel.as<float4>();
   t.node_mask = s->node_mask.as<uint32_t>();
+  if (!s->seen) {
+    void* q = nullptr;
+    if (hipHostMalloc(&q, 2 * sizeof(uint32_t), hipHostMallocDefault) == hipSuccess) s->seen = static_cast<uint32_t*>(q);
+    else (void)hipGetLastError();  // launches then follow the synchronized counts only
+    s->forget_seen();
+  }
+  t.seen = s->seen;
   s->p2g_blocks = std::min<uint32_t>(pblock_cap, 65535);
   s->topo_valid = false;
   s->table_dirty = true;
@@ -1742,6 +1761,7 @@ tmpm_status prepare_packed(tmpm_session* s, PackedParticles& pk) {
   // topology capacity from the initial block counts, with headroom
   uint64_t pblocks = 0, gblocks = 0;
   count_blocks(pk.pos32, pk.region, pk.inv_h, pblocks, gblocks);
+  s->forget_seen();
   s->last_pblocks = (uint32_t)pblocks;
   s->last_gblocks = (uint32_t)gblocks;
   // CPIC splits blocks that straddle a triangle by side: more headroom
@@ -1851,17 +1871,17 @@ uint32_t particles_per_block(const tmpm_session* s) {
 //         11.8;  503 of 239: 38 / 25.3 / 16.2 / 13.2;  716 of 70: 18.5 / 14.2 /
 //         10.6 / 15.4;  900 of 278: 43.8 / 29.7 / 20.3 / 22.6.
 uint32_t widened_p2g(const tmpm_session* s, uint32_t threads, int copies) {
-  const uint32_t b = s->last_pblocks;
+  const uint32_t b = s->pblocks_now();
   if (threads != 128 || copies != 1 || b > 4 * kCus) return threads;
   return b <= 2 * kCus ? 512u : 256u;
 }
 uint32_t widened_g2p(const tmpm_session* s, uint32_t threads) {
-  return threads == 256 && !s->plastic && !s->shapes && s->last_pblocks <= 2 * kCus ? 512u : threads;
+  return threads == 256 && !s->plastic && !s->shapes && s->pblocks_now() <= 2 * kCus ? 512u : threads;
 }
 
 // Workgroups of a launch that takes one block each (every kernel strides over
-// the rest): an eighth more than the last synchronized count, in steps of an
-// eighth, so that a captured plan holds for a while.  Launched for the whole
+// the rest): an eighth more than the last count the host has (pblocks_now), in
+// steps of an eighth, so that a captured plan holds for a while.  Launched for the whole
 // capacity, four times the blocks at the start, three of four workgroups
 // found no block.
 uint32_t launch_blocks(uint32_t last, uint32_t most) {
@@ -2035,8 +2055,8 @@ SubstepPlan plan_substep(tmpm_session* s, bool apply_force, bool first, bool mor
   pl.body_scene = s->body_scene.as<uint32_t>();
   pl.obstacle_total = s->obstacle_total;
   pl.body_total = s->body_total;
-  pl.pblocks = launch_blocks(s->last_pblocks, s->p2g_blocks);
-  pl.gblocks = launch_blocks(s->last_gblocks, s->topo.grid_cap);
+  pl.pblocks = launch_blocks(s->pblocks_now(), s->p2g_blocks);
+  pl.gblocks = launch_blocks(s->gblocks_now(), s->topo.grid_cap);
   effective_p2g_shape(s, pl.p2g_threads, pl.copies);
   pl.p2g_threads = widened_p2g(s, pl.p2g_threads, pl.copies);
   pl.g2p_threads = widened_g2p(s, effective_g2p_threads(s));
@@ -3330,6 +3350,7 @@ tmpm_status tmpm_session_synchronize(tmpm_session* s) {
       const uint32_t global = s->batch ? (counters[CNT_ERROR] & (ERR_TOPOLOGY | ERR_INTERNAL)) : counters[CNT_ERROR];
       tmpm_status st = status_from_error_bits(global);
       if (st != TMPM_OK) return st;
+      s->forget_seen();
       s->last_pblocks = counters[CNT_PARTICLE_BLOCKS];
       s->last_gblocks = counters[CNT_GRID_BLOCKS];
       if (counters[CNT_REACT_SATURATED]) {

@@ -73,3 +73,28 @@ def test_blocks_that_multiply_between_synchronizations(transfers, mode):
     assert ta == tb and ta["particle_blocks"] > 72  # 72: the grid launched for one block
     for name in ("position", "velocity", "affine", "deformation"):
         assert np.array_equal(getattr(a, name), getattr(b, name)), name
+
+
+@pytest.mark.parametrize("graphs", ["0", "1"])
+def test_launches_follow_full_binnings_without_a_synchronize(transfers, graphs, monkeypatch):
+    # one block becomes hundreds over submissions that nothing waits for: the launch widths and
+    # grids change on the way, the state does not
+    rng = np.random.default_rng(3)
+    pos = (16.6 + rng.uniform(0.0, 3.8, size=(3000, 3))) * H
+    vel = (pos - 18.5 * H) * 0.1 / DT
+    m = MaterialModel.fluid(1.0e-3, 7.0, 0.0)
+    monkeypatch.setenv("TMPM_GRAPHS", graphs)
+    runs = []
+    for wait in (False, True):
+        s = HipMpmResidentSession(transfers, world_of(pos, vel, m), DT, "fp32")
+        for _ in range(34):
+            s.submit_steps(3)
+            if wait:
+                s.synchronize()
+        s.synchronize()
+        runs.append((s.read_particles(), s.topology_stats()))
+        s.close()
+    (a, ta), (b, tb) = runs
+    assert ta == tb and ta["particle_blocks"] > 512
+    for name in ("position", "velocity", "affine", "deformation"):
+        assert np.array_equal(getattr(a, name), getattr(b, name)), name

@@ -125,6 +125,7 @@ struct DevObstacle {
 constexpr int kMaxConvexPlanes = 128;  // planes per convex obstacle (gpu.rs pack_obstacle)
 constexpr int kGatherFloats = 29;    // per particle in a scene gather (k_gather_scene)
 constexpr int kReadbackHeader = 16;  // words before the records of k_gather_state
+constexpr int kReadbackFlags = 14;   // two of them: "not finite" of the even and of the odd readbacks
 
 // Rigid body state (GpuRigidBodyState, phys/src/gpu_rigid_state.rs:17-28):
 // position and inverse mass, XYZW orientation, world velocities, body-frame

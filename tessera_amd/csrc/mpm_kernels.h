@@ -43,7 +43,7 @@ void launch_retire(const Parts& p, uint32_t first, uint32_t count, hipStream_t s
 void launch_renumber(uint32_t* ins_id, uint32_t n, uint32_t first, uint32_t count, hipStream_t s);
 void launch_gather_scene(const Parts& p, uint32_t first, uint32_t count, float* out, hipStream_t s);
 // header and records (k_gather_state): kReadbackHeader + kGatherFloats for each of `count` insertion indices
-void launch_gather_state(const Parts& p, const DevClass* c, const Topo& t, uint32_t mark, uint32_t count, float* out,
+void launch_gather_state(const Parts& p, const DevClass* c, const Topo& t, uint32_t turn, uint32_t count, float* out,
                          hipStream_t s);
 void launch_copy(const float4* src, float4* dst, size_t n, hipStream_t s);
 // flags[c] = 1 for lattice candidate c (x-major, then y, then z) inside the closed mesh

@@ -2750,21 +2750,26 @@ __global__ __launch_bounds__(256) void k_gather_scene(Parts p, uint32_t first, u
 }
 
 // A plain session's readback: kReadbackHeader words (the counters, the scene's
-// error bits, and `mark` in the last one if a particle that moves is not
+// error bits, and at kReadbackFlags + turn whether a particle that moves is not
 // finite), then every particle's record by insertion index, in one buffer for
-// one copy to the host.
+// one copy to the host.  `turn` is 0 and 1 in turn: each launch clears the flag
+// of the next one, whose workgroups run in no order, and the host clears both
+// where it allocates the buffer.
 __global__ __launch_bounds__(256) void k_gather_state(Parts p, const DevClass* classes, const uint32_t* counters,
-                                                      const uint32_t* scene_err, uint32_t mark, uint32_t count,
+                                                      const uint32_t* scene_err, uint32_t turn, uint32_t count,
                                                       float* out) {
   uint32_t* header = reinterpret_cast<uint32_t*>(out);
   if (blockIdx.x == 0 && threadIdx.x < CNT_COUNT) header[threadIdx.x] = counters[threadIdx.x];
-  if (blockIdx.x == 0 && threadIdx.x == CNT_COUNT) header[CNT_COUNT] = scene_err[0];
+  if (blockIdx.x == 0 && threadIdx.x == CNT_COUNT) {
+    header[CNT_COUNT] = scene_err[0];
+    header[kReadbackFlags + 1 - turn] = 0;
+  }
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < p.n; i += gridDim.x * blockDim.x) {
     const uint32_t g = p.ins_id[i];
     if (g >= count) continue;  // kInvalid: no particle in the slot
     bool finite;
     gather_record(p, i, out + kReadbackHeader + (size_t)g * kGatherFloats, finite);
-    if (!finite && !classes[p.cls[i]].fixed) header[kReadbackHeader - 1] = mark;
+    if (!finite && !classes[p.cls[i]].fixed) header[kReadbackFlags + turn] = 1;
   }
 }
 
@@ -3221,9 +3226,9 @@ void launch_renumber(uint32_t* ins_id, uint32_t n, uint32_t first, uint32_t coun
 void launch_gather_scene(const Parts& p, uint32_t first, uint32_t count, float* out, hipStream_t s) {
   hipLaunchKernelGGL(k_gather_scene, dim3(grid_for(p.n, 256, 8192)), dim3(256), 0, s, p, first, count, out);
 }
-void launch_gather_state(const Parts& p, const DevClass* c, const Topo& t, uint32_t mark, uint32_t count, float* out,
+void launch_gather_state(const Parts& p, const DevClass* c, const Topo& t, uint32_t turn, uint32_t count, float* out,
                          hipStream_t s) {
-  hipLaunchKernelGGL(k_gather_state, dim3(grid_for(p.n, 256, 8192)), dim3(256), 0, s, p, c, t.counters, t.scene_err, mark,
+  hipLaunchKernelGGL(k_gather_state, dim3(grid_for(p.n, 256, 8192)), dim3(256), 0, s, p, c, t.counters, t.scene_err, turn,
                      count, out);
 }
 void launch_audit(const Parts& p, const DevClass* c, double* out, hipStream_t s) {

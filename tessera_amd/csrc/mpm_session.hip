@@ -626,7 +626,7 @@ struct tmpm_session {
   ParticleBuffers synced;
   uint32_t synced_n = 0;
   DevBuf staging;
-  uint32_t readback_mark = 0;
+  uint32_t readback_turn = 0;  // of the next k_gather_state: 0, 1
   DevBuf disabled_rec;     // snapshot records of disabled particles (2 float4 each)
   std::vector<float4> disabled_host;
   PackedParticles stage;                // admission staging, reused
@@ -2368,11 +2368,14 @@ tmpm_status read_back(tmpm_session* s, uint32_t counters[CNT_COUNT], F&& check) 
   }
   if (hipSetDevice(s->ctx->device) != hipSuccess) return fail(TMPM_READBACK, "cannot select device");
   const size_t n = scene.count, words = kReadbackHeader + n * kGatherFloats;
-  if (s->staging.bytes < 4 * words) HIP_TRY(s->staging.alloc(4 * words));
-  const uint32_t mark = ++s->readback_mark | 0x80000000u;
+  if (s->staging.bytes < 4 * words) {  // a plain session uses it for nothing else
+    HIP_TRY(s->staging.alloc(4 * words));
+    HIP_TRY(hipMemsetAsync(s->staging.ptr, 0, 4 * kReadbackHeader, s->stream));
+  }
+  const uint32_t turn = s->readback_turn;
+  s->readback_turn = 1 - turn;
   float* dev = s->staging.as<float>();
-  launch_gather_state(s->parts(s->cur), s->classes.as<DevClass>(), s->topo, mark, (uint32_t)n, dev,
-                      s->stream);
+  launch_gather_state(s->parts(s->cur), s->classes.as<DevClass>(), s->topo, turn, (uint32_t)n, dev, s->stream);
   HIP_TRY(hipGetLastError());
   // pieces of whole records; the first one has the header
   const size_t per = (ReadbackPool::kBytes / 4 - kReadbackHeader) / kGatherFloats;
@@ -2403,7 +2406,7 @@ tmpm_status read_back(tmpm_session* s, uint32_t counters[CNT_COUNT], F&& check) 
       if (k == 0) {
         const uint32_t* header = reinterpret_cast<const uint32_t*>(data);
         std::memcpy(counters, header, 4 * CNT_COUNT);
-        tmpm_status st = check(header[CNT_COUNT], header[kReadbackHeader - 1] == mark);
+        tmpm_status st = check(header[CNT_COUNT], header[kReadbackFlags + turn] != 0);
         if (st != TMPM_OK) return st;
         data += kReadbackHeader;
       }

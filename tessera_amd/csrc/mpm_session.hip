@@ -24,7 +24,6 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <tuple>
 #include <unordered_map>
@@ -32,6 +31,7 @@
 
 #include "../../include/tessera_mpm.h"
 #include "mpm_device.h"
+#include "mpm_host.h"
 #include "mpm_kernels.h"
 
 using namespace tmpm;
@@ -185,37 +185,6 @@ inline bool cell_f32(float x, float inv_h, int32_t& c) {
 // ---------------------------------------------------------------------------
 // Host world (f64, insertion order) — `MpmWorld` (world.rs:206-221).
 // ---------------------------------------------------------------------------
-// Runs fn(begin, end) over [0, n) in up to 16 host threads (chunks of at
-// least min_chunk items; small ranges run inline).  Used for the per-particle
-// host work of uploads and admissions.
-template <class F>
-void parallel_for(size_t n, F&& fn, size_t min_chunk = 16384) {
-  const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-  const size_t chunks = std::min<size_t>(hw, (n + min_chunk - 1) / min_chunk);
-  if (chunks <= 1) {
-    fn((size_t)0, n);
-    return;
-  }
-  const size_t step = (n + chunks - 1) / chunks;
-  std::vector<std::thread> pool;
-  pool.reserve(chunks);
-  size_t inline_from = chunks;  // chunks no thread could be started for run here
-  for (size_t c = 1; c < chunks; ++c) {
-    const size_t b = c * step, e = std::min(n, b + step);
-    if (b >= e) break;
-    try {
-      pool.emplace_back([&fn, b, e] { fn(b, e); });
-    } catch (const std::system_error&) {
-      inline_from = c;
-      break;
-    }
-  }
-  fn((size_t)0, std::min(n, step));
-  for (size_t c = inline_from; c < chunks; ++c)
-    if (c * step < n) fn(c * step, std::min(n, c * step + step));
-  for (auto& t : pool) t.join();
-}
-
 struct OwnedObstacle {
   tmpm_obstacle o;
   std::vector<double> planes;
@@ -627,6 +596,7 @@ struct tmpm_session {
   uint32_t synced_n = 0;
   DevBuf staging;
   uint32_t readback_turn = 0;  // of the next k_gather_state: 0, 1
+  StateColumns<DVec> spare_columns;  // of a readback in pieces
   DevBuf disabled_rec;     // snapshot records of disabled particles (2 float4 each)
   std::vector<float4> disabled_host;
   PackedParticles stage;                // admission staging, reused
@@ -2320,52 +2290,22 @@ struct ReadbackBuffers {
   }
 };
 
-// Records [first, first + count) of a k_gather_state buffer into the world
-// (gpu.rs:2295-2329 apply_gpu_transfers): f32 widened to f64.  Forces are
-// one-shot; fixed particles end with zero v and C (world.rs:419-430).
-void widen_records(HostWorld& w, const float* rec, size_t first, size_t count, bool records, bool plastic) {
-  parallel_for(count, [&](size_t b, size_t e) {
-    for (size_t k = b; k < e; ++k) {
-      const size_t i = first + k;
-      w.force[3 * i] = w.force[3 * i + 1] = w.force[3 * i + 2] = 0.0;
-      if (!w.enabled[i]) continue;
-      if (w.fixed[i]) {
-        for (int q = 0; q < 3; ++q) w.vel[3 * i + q] = 0.0;
-        for (int q = 0; q < 9; ++q) w.C[9 * i + q] = 0.0;
-        continue;
-      }
-      if (!records) continue;
-      const float* r = rec + k * kGatherFloats;
-      for (int q = 0; q < 3; ++q) {
-        w.pos[3 * i + q] = r[q];
-        w.vel[3 * i + q] = r[4 + q];
-      }
-      for (int q = 0; q < 9; ++q) {
-        w.C[9 * i + q] = r[8 + q];
-        w.F[9 * i + q] = r[17 + q];
-      }
-      if (plastic && is_plastic(w.material[i]))
-        for (int q = 0; q < 3; ++q) w.plastic[3 * i + q] = r[26 + q];
-    }
-  });
-}
+static_assert(kRecordFloats == (size_t)kGatherFloats, "the records of k_gather_state");
 
 // A plain session's readback: one kernel lays the counters and every
 // particle's record out in insertion order, one copy (in pieces, of which the
 // host widens one while the next is copied) brings them to page-locked memory.
 // `check` sees the counters and scene error bits before the world is touched;
-// a status other than TMPM_OK ends the readback.  The host spent 8.2 ms on
-// 59,319 particles with a copy per column, two copies of the world and a
-// serial scatter.
+// a status other than TMPM_OK, its own or of a later piece, ends the readback
+// and leaves the world as it was.  The host spent 8.2 ms on 59,319 particles
+// with a copy per column, two copies of the world and a serial scatter.
 template <class F>
 tmpm_status read_back(tmpm_session* s, uint32_t counters[CNT_COUNT], F&& check) {
   SceneState& scene = s->scenes[0];
   HostWorld& w = scene.world;
-  if (!s->prepared) {
-    tmpm_status st = check(0u, false);
-    if (st == TMPM_OK) widen_records(w, nullptr, 0, w.size(), false, false);
-    return st;
-  }
+  if (!s->prepared)
+    return (tmpm_status)read_pieces(w, s->spare_columns, w.size(), std::max<size_t>(w.size(), 1), false, is_plastic,
+                                    [&](size_t, const float*&) -> int { return check(0u, false); });
   if (hipSetDevice(s->ctx->device) != hipSuccess) return fail(TMPM_READBACK, "cannot select device");
   const size_t n = scene.count, words = kReadbackHeader + n * kGatherFloats;
   if (s->staging.bytes < 4 * words) {  // a plain session uses it for nothing else
@@ -2394,26 +2334,20 @@ tmpm_status read_back(tmpm_session* s, uint32_t counters[CNT_COUNT], F&& check) 
   struct Drain {
     hipStream_t s;
     ~Drain() { (void)hipStreamSynchronize(s); }
-  };
-  {
-    Drain drain{s->stream};
-    hipError_t e = copy(0);
-    for (size_t k = 0; k < pieces; ++k) {
-      if (e == hipSuccess && k + 1 < pieces) e = copy(k + 1);
-      if (e == hipSuccess) e = hipEventSynchronize(buf.b[k & 1]->copied);
-      if (e != hipSuccess) return fail(TMPM_READBACK, std::string("device failure: ") + hipGetErrorString(e));
-      const float* data = buf.b[k & 1]->mem.data();
-      if (k == 0) {
-        const uint32_t* header = reinterpret_cast<const uint32_t*>(data);
-        std::memcpy(counters, header, 4 * CNT_COUNT);
-        tmpm_status st = check(header[CNT_COUNT], header[kReadbackFlags + turn] != 0);
-        if (st != TMPM_OK) return st;
-        data += kReadbackHeader;
-      }
-      widen_records(w, data, k * per, std::min(n - k * per, per), true, s->plastic);
-    }
-  }
-  return TMPM_OK;
+  } drain{s->stream};
+  hipError_t e = copy(0);
+  return (tmpm_status)read_pieces(w, s->spare_columns, n, per, s->plastic, is_plastic,
+                                  [&](size_t k, const float*& rec) -> int {
+    if (e == hipSuccess && k + 1 < pieces) e = copy(k + 1);
+    if (e == hipSuccess) e = hipEventSynchronize(buf.b[k & 1]->copied);
+    if (e != hipSuccess) return fail(TMPM_READBACK, std::string("device failure: ") + hipGetErrorString(e));
+    rec = buf.b[k & 1]->mem.data();
+    if (k > 0) return TMPM_OK;
+    const uint32_t* header = reinterpret_cast<const uint32_t*>(rec);
+    std::memcpy(counters, header, 4 * CNT_COUNT);
+    rec += kReadbackHeader;
+    return check(header[CNT_COUNT], header[kReadbackFlags + turn] != 0);
+  });
 }
 
 // Batches: brings scene k's host world up to its last synchronize by

@@ -717,8 +717,15 @@ __device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, cons
                                              const DevScene* scenes) {
   __shared__ uint32_t s_new, s_slots, s_rest;
   const uint32_t strays = min(t.counters[CNT_STRAYS], p.n);
-  if (strays == 0) return;
   const uint32_t tid = threadIdx.x;
+  // A batch scene that failed in an earlier substep is not binned any more
+  // (see k_bin_insert); on the lists its particles still are, so P2G drops
+  // those of the scenes marked here.  Scenes that fail in this substep's P2G
+  // are not marked: they run it to its end, as after a full binning.
+  if (t.isolate && (t.counters[CNT_ERROR] & (ERR_RESIDENT | ERR_FIXED_RANGE)) != 0u)
+    for (uint32_t s = tid; s < t.scene_total; s += kUpdateThreads)
+      if (t.scene_err[s] != 0u) t.scene_err[s] |= ERR_STOPPED;
+  if (strays == 0) return;
   const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS], ng = t.counters[CNT_GRID_BLOCKS],
                  binned = t.counters[CNT_BINNED];
   if (tid == 0) s_new = s_slots = s_rest = 0;
@@ -730,7 +737,7 @@ __device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, cons
     const uint32_t i = e.x;
     const DevClass& c = classes[p.cls[i]];
     uint32_t b = kInvalid;
-    // as in k_bin_insert, a failed scene's particles are not binned any more
+    // a failed scene makes no blocks any more, as in k_bin_insert
     int3 cell;
     if (!(t.isolate && t.scene_err[c.region >> 16] != 0u) && cell3(p.pos_mass[i], c.inv_h, cell)) {
       bool claimed;
@@ -1858,12 +1865,18 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS
     }
     const int4 key = uniform4(t.grid_key[own]);
     const DevScene& sc = scenes[(uint32_t)key.w >> 16];
+    // A scene that k_bin_update found failed: the block takes part in nothing
+    // more in this substep, here and in G2P (which finds its list empty).
+    const bool stopped =
+        t.listed && t.isolate && (uniform1(t.scene_err[(uint32_t)key.w >> 16]) & ERR_STOPPED) != 0u;
+    const uint32_t todo = stopped ? 0u : total;
+    if (stopped && tid == 0) t.cur.meta[k] = make_uint4(0, 0, 0, 0);
     const float h = sc.h, inv_h = sc.inv_h;
     const float stress_scale = -sc.dt * sc.inv_d;
     const float mscale = exp2f((float)sc.mass_shift), pscale = exp2f((float)sc.mom_shift);
     const int ox = key.x * kBlockCells, oy = key.y * kBlockCells, oz = key.z * kBlockCells;
-    bool bad = false, range = total - list.holes > kP2GMaxBlock;
-    for (uint32_t j = tid; j < total; j += THREADS) {
+    bool bad = false, range = !stopped && total - list.holes > kP2GMaxBlock;
+    for (uint32_t j = tid; j < todo; j += THREADS) {
       const uint32_t i = j == (uint32_t)tid               ? i_first
                          : j == (uint32_t)(tid + THREADS) ? i_second
                                                           : block_particle(list, j);

@@ -2324,7 +2324,11 @@ __global__ __launch_bounds__(!SHAPES && !PLASTIC ? 512 : 256) __attribute__((amd
         const int lx = cell.x - ox, ly = cell.y - oy, lz = cell.z - oz;
         if ((unsigned)lx > 3u || (unsigned)ly > 3u || (unsigned)lz > 3u) {
           bad = true;
-          if (move) {  // binning disagrees with this block: keep the particle as it was
+          if (move) {  // binning disagrees with this block: keep the particle as it was, on no list
+            if (t.build) {
+              t.nxt.idx[w + (uint64_t)kListRoom * k] = kInvalid;
+              atomicAdd(&s_left, 1u);
+            }
             o.pos_mass[w] = pm;
             o.vel_vol[w] = p.vel_vol[i];
 #pragma unroll
@@ -2428,6 +2432,7 @@ __global__ __launch_bounds__(!SHAPES && !PLASTIC ? 512 : 256) __attribute__((amd
                     nb.x > sc.last_base[0] || nb.y > sc.last_base[1] || nb.z > sc.last_base[2];
           if (MOVE && t.build && !ok) {
             t.nxt.idx[w + (uint64_t)kListRoom * k] = kInvalid;
+            atomicAdd(&s_left, 1u);
           } else if (t.build && ok) {
             const int dx = (nb.x >> 2) - key.x, dy = (nb.y >> 2) - key.y, dz = (nb.z >> 2) - key.z;
             if ((dx | dy | dz) != 0 || !list_stay(w)) list_later(w, dx, dy, dz);

@@ -702,9 +702,10 @@ __global__ __launch_bounds__(256) void k_bin_scatter(Parts p, Topo t) {
 // into the table, the first stray of each new particle block takes the next
 // id, the 7 upper neighbours of the new blocks go into the table, and the
 // tiles' slots and the lists are filled.  Blocks that particles have left stay
-// until the next full binning; their tiles are zero.  Every sum runs over the
-// same particles as after a full binning, in integers, so results are the same
-// bit for bit.
+// until the next full binning; their tiles are zero.  Where they leave no room
+// for a new one, the blocks are made anew from the particles (rebuild_lists).
+// Every sum runs over the same particles as after a full binning, in integers,
+// so results are the same bit for bit.
 //
 // In a kernel trace the four binning kernels took 39 us of a substep of 153 us
 // at 1M particles, 96 of 576 us at 4M and 19 of 52 us at 8k; this launch takes
@@ -713,9 +714,130 @@ __global__ __launch_bounds__(256) void k_bin_scatter(Parts p, Topo t) {
 constexpr int kUpdateThreads = 512;
 constexpr uint32_t kClaimed = kInvalid - 1;  // bucket_pblock of a block whose id is being taken
 
-__device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, const DevClass* classes,
+// A barrier after which every thread of the workgroup sees what the others
+// wrote before it, also where device-scope atomics went past this CU's cache.
+__device__ __forceinline__ void phase_end() {
+  __threadfence();
+  __syncthreads();
+  __threadfence();
+}
+
+// The blocks and lists of this substep made anew by one workgroup, with no
+// block that holds no particle: what kernels 1-4 do over the whole chip, for
+// the rare substep whose visited blocks (a fast, thin scene) do not fit beside
+// the emptied ones, though a full binning of it would.  Whatever update_lists
+// had begun is dropped.
+__device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, const DevClass* classes,
+                                              const DevScene* scenes) {
+  __shared__ uint32_t s_blocks, s_tiles, s_sum[kUpdateThreads];
+  const uint32_t tid = threadIdx.x;
+  const uint32_t room = min(t.pblock_room, t.grid_room);  // a block's grid slot is its id
+  if (tid == 0) s_blocks = s_tiles = 0;
+  bool over = false;
+  phase_end();
+  for (uint32_t b = tid; b <= t.bucket_mask; b += kUpdateThreads) {
+    t.owner[b] = 0;
+    t.bucket_count[b] = 0;
+    t.bkey[b].x = kNoKey;
+    t.bucket_pblock[b] = t.bucket_slot[b] = kInvalid;
+  }
+  phase_end();
+  for (uint32_t i = tid; i < p.n; i += kUpdateThreads) {
+    const float4 pm = p.pos_mass[i];
+    const DevClass& c = classes[p.cls[i]];
+    uint32_t b = kInvalid;
+    int3 cell;
+    if (pm.w > 0.0f && !(t.isolate && t.scene_err[c.region >> 16] != 0u) && cell3(pm, c.inv_h, cell)) {
+      bool claimed;
+      const int4 key = make_int4(cell.x >> 2, cell.y >> 2, cell.z >> 2, (int)c.region);
+      b = hash_insert(p, t, classes, scenes, key, i + 1, claimed);
+      if (b == kInvalid) {
+        over = true;
+      } else {
+        t.prank[i] = atomicAdd(&t.bucket_count[b], 1u);
+        if (claimed) {
+          const uint32_t k = atomicAdd(&s_blocks, 1u);
+          if (k < room) {
+            t.pblock_nbr[8 * k] = b;
+            t.bucket_pblock[b] = t.bucket_slot[b] = k;
+            t.grid_key[k] = key;
+            clear_rev(t, k);
+          } else {
+            over = true;
+          }
+        }
+      }
+    }
+    t.pslot[i] = b;
+  }
+  phase_end();
+  const uint32_t npb = min(s_blocks, room);
+  for (uint32_t q = tid; q < 7 * npb; q += kUpdateThreads) {
+    const uint32_t k = q / 7u, d = q % 7u + 1u, b = t.pblock_nbr[8 * k];
+    int4 key = t.grid_key[k];
+    key.x += (int)(d >> 2);
+    key.y += (int)((d >> 1) & 1);
+    key.z += (int)(d & 1);
+    bool claimed;
+    const uint32_t got = hash_insert<false, true>(p, t, classes, scenes, key, p.n + 1 + 8 * b + d, claimed);
+    if (got == kInvalid) {
+      over = true;
+    } else if (claimed) {
+      const uint32_t slot = npb + atomicAdd(&s_tiles, 1u);
+      if (slot < t.grid_room) {
+        t.bucket_slot[got] = slot;
+        t.grid_key[slot] = key;
+        clear_rev(t, slot);
+      } else {
+        over = true;
+      }
+    }
+    t.pblock_nbr[8 * k + d] = got;
+  }
+  phase_end();
+  for (uint32_t q = tid; q < 8 * npb; q += kUpdateThreads) {
+    const uint32_t b = t.pblock_nbr[q], slot = b == kInvalid ? kInvalid : t.bucket_slot[b];
+    t.pblock_slot8[q] = slot;
+    if (slot != kInvalid) t.grid_rev[8 * slot + (q & 7)] = q >> 3;
+  }
+  // where each block's particles start, in id order: a run of blocks per thread
+  const uint32_t run = (npb + kUpdateThreads - 1) / kUpdateThreads;
+  const uint32_t k0 = min(tid * run, npb), k1 = min(k0 + run, npb);
+  uint32_t sum = 0;
+  for (uint32_t k = k0; k < k1; ++k) sum += t.bucket_count[t.pblock_nbr[8 * k]];
+  s_sum[tid] = sum;
+  phase_end();
+  uint32_t at = 0, binned = 0;
+  for (uint32_t u = 0; u < kUpdateThreads; ++u) {
+    if (u < tid) at += s_sum[u];
+    binned += s_sum[u];
+  }
+  for (uint32_t k = k0; k < k1; ++k) {
+    const uint32_t len = t.bucket_count[t.pblock_nbr[8 * k]];
+    t.pblock_start[k] = at;
+    t.pblock_len[k] = len;
+    t.cur.meta[k] = make_uint4(len, 0, 0, 0);
+    at += len;
+  }
+  phase_end();
+  for (uint32_t i = tid; i < p.n; i += kUpdateThreads) {
+    const uint32_t b = t.pslot[i], k = b == kInvalid ? kInvalid : t.bucket_pblock[b];
+    if (k != kInvalid) t.cur.idx[t.pblock_start[k] + (uint64_t)t.cur.pitch * k + t.prank[i]] = i;
+  }
+  flag_error(t.counters, over, ERR_TOPOLOGY);
+  if (tid == 0) {
+    t.counters[CNT_PARTICLE_BLOCKS] = npb;
+    t.counters[CNT_GRID_BLOCKS] = min(npb + s_tiles, t.grid_room);
+    t.counters[CNT_BINNED] = binned;
+    t.counters[CNT_STRAYS] = 0;
+  }
+}
+
+// Whether there is no room for the new blocks: rebuild_lists has to follow.
+// Uniform over the workgroup.
+__device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, const DevClass* classes,
                                              const DevScene* scenes) {
-  __shared__ uint32_t s_new, s_slots, s_rest;
+  __shared__ uint32_t s_new, s_slots, s_rest, s_over;
   const uint32_t strays = min(t.counters[CNT_STRAYS], p.n);
   const uint32_t tid = threadIdx.x;
   // A batch scene that failed in an earlier substep is not binned any more
@@ -725,11 +847,25 @@ __device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, cons
   if (t.isolate && (t.counters[CNT_ERROR] & (ERR_RESIDENT | ERR_FIXED_RANGE)) != 0u)
     for (uint32_t s = tid; s < t.scene_total; s += kUpdateThreads)
       if (t.scene_err[s] != 0u) t.scene_err[s] |= ERR_STOPPED;
-  if (strays == 0) return;
+  if (strays == 0) return false;
   const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS], ng = t.counters[CNT_GRID_BLOCKS],
                  binned = t.counters[CNT_BINNED];
-  if (tid == 0) s_new = s_slots = s_rest = 0;
+  if (tid == 0) s_new = s_slots = s_rest = s_over = 0;
+  __syncthreads();
+  // No room: what is left of the phases is skipped (inserts beyond it would fill
+  // the table, and each then probes all of it).
   bool over = false;
+  auto no_room = [&] { over = *(volatile uint32_t*)&s_over != 0u || over; return over; };
+  auto overflow = [&] { over = true; *(volatile uint32_t*)&s_over = 1u; };
+  // grid slot of a new bucket
+  auto take_slot = [&](uint32_t b, int4 key) {
+    const uint32_t slot = ng + atomicAdd(&s_slots, 1u);
+    t.bucket_pblock[b] = t.bucket_slot[b] = kInvalid;
+    if (slot >= t.grid_room) return overflow();
+    t.bucket_slot[b] = slot;
+    t.grid_key[slot] = key;
+    clear_rev(t, slot);
+  };
   // the buckets of the particles whose block is to be looked up (pslot: kInvalid for none)
   for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
     const uint2 e = t.stray[s];
@@ -739,27 +875,16 @@ __device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, cons
     uint32_t b = kInvalid;
     // a failed scene makes no blocks any more, as in k_bin_insert
     int3 cell;
-    if (!(t.isolate && t.scene_err[c.region >> 16] != 0u) && cell3(p.pos_mass[i], c.inv_h, cell)) {
+    if (!no_room() && !(t.isolate && t.scene_err[c.region >> 16] != 0u) && cell3(p.pos_mass[i], c.inv_h, cell)) {
       bool claimed;
-      b = hash_insert<false, true>(p, t, classes, scenes,
-                                   make_int4(cell.x >> 2, cell.y >> 2, cell.z >> 2, (int)c.region), i + 1, claimed);
-      if (b == kInvalid) over = true;
-      else if (claimed) t.bucket_pblock[b] = t.bucket_slot[b] = kInvalid;
+      const int4 key = make_int4(cell.x >> 2, cell.y >> 2, cell.z >> 2, (int)c.region);
+      b = hash_insert<false, true>(p, t, classes, scenes, key, i + 1, claimed);
+      if (b == kInvalid) overflow();
+      else if (claimed) take_slot(b, key);
     }
     t.pslot[i] = b;
   }
-  __syncthreads();
-  // grid slot of a bucket that has none
-  auto take_slot = [&](uint32_t b) {
-    const uint32_t slot = ng + atomicAdd(&s_slots, 1u);
-    if (slot >= t.grid_room) {
-      over = true;
-      return;
-    }
-    t.bucket_slot[b] = slot;
-    t.grid_key[slot] = t.bkey[b];
-    clear_rev(t, slot);
-  };
+  if (__syncthreads_or(over)) return true;
   // new particle blocks: the first stray of each takes its id
   for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
     const uint2 e = t.stray[s];
@@ -767,18 +892,17 @@ __device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, cons
     if (b == kInvalid || atomicCAS(&t.bucket_pblock[b], kInvalid, kClaimed) != kInvalid) continue;
     const uint32_t pb = npb + atomicAdd(&s_new, 1u);
     if (pb >= t.pblock_room) {
-      over = true;
+      overflow();
       continue;
     }
-    if (t.bucket_slot[b] == kInvalid) take_slot(b);
     t.pblock_nbr[8 * pb] = b;
     t.pblock_start[pb] = binned;
     t.pblock_len[pb] = 0;
     t.cur.meta[pb] = make_uint4(0, 0, 0, 0);
     t.bucket_pblock[b] = pb;
   }
-  __syncthreads();
-  const uint32_t made = min(s_new, t.pblock_room - npb);
+  if (__syncthreads_or(over)) return true;
+  const uint32_t made = s_new;
   for (uint32_t q = tid; q < 7 * made; q += kUpdateThreads) {
     const uint32_t pb = npb + q / 7u, d = q % 7u + 1u;
     const uint32_t b = t.pblock_nbr[8 * pb];
@@ -786,17 +910,14 @@ __device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, cons
     k.x += (int)(d >> 2);
     k.y += (int)((d >> 1) & 1);
     k.z += (int)(d & 1);
-    bool claimed;
-    const uint32_t got = hash_insert<false, true>(p, t, classes, scenes, k, p.n + 1 + 8 * b + d, claimed);
-    if (got == kInvalid) {
-      over = true;
-    } else if (claimed) {
-      t.bucket_pblock[got] = t.bucket_slot[got] = kInvalid;
-      take_slot(got);
-    }
+    bool claimed = false;
+    const uint32_t got =
+        no_room() ? kInvalid : hash_insert<false, true>(p, t, classes, scenes, k, p.n + 1 + 8 * b + d, claimed);
+    if (got == kInvalid) overflow();
+    else if (claimed) take_slot(got, k);
     t.pblock_nbr[8 * pb + d] = got;
   }
-  __syncthreads();
+  if (__syncthreads_or(over)) return true;
   for (uint32_t q = tid; q < 8 * made; q += kUpdateThreads) {
     const uint32_t pb = npb + (q >> 3), d = q & 7, b = t.pblock_nbr[8 * pb + d];
     const uint32_t slot = b == kInvalid ? kInvalid : t.bucket_slot[b];
@@ -809,10 +930,6 @@ __device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, cons
     const uint32_t i = e.x, b = e.y == kInvalid ? t.pslot[i] : kInvalid;
     if (b == kInvalid) continue;
     const uint32_t pb = t.bucket_pblock[b];
-    if (pb >= t.pblock_room) {  // no room for the block (flagged)
-      t.bucket_pblock[b] = kInvalid;
-      continue;
-    }
     const uint32_t pos = atomicAdd(&t.cur.meta[pb].y, 1u);
     if (pos < kListRoom) {
       t.cur.idx[t.list_came + (uint64_t)kListRoom * pb + pos] = i;
@@ -836,12 +953,17 @@ __device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, cons
     if (at < p.n) t.cur.idx[t.list_rest + at] = e.x;
     else atomicOr(&t.counters[CNT_ERROR], ERR_INTERNAL);  // more entries than particles: never write past them
   }
-  flag_error(t.counters, over, ERR_TOPOLOGY);
   if (tid == 0) {
     t.counters[CNT_PARTICLE_BLOCKS] = npb + made;
-    t.counters[CNT_GRID_BLOCKS] = min(ng + s_slots, t.grid_room);
+    t.counters[CNT_GRID_BLOCKS] = ng + s_slots;
     t.counters[CNT_STRAYS] = 0;
   }
+  return false;
+}
+
+__device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, const DevClass* classes,
+                                             const DevScene* scenes) {
+  if (extend_lists(p, t, classes, scenes)) rebuild_lists(p, t, classes, scenes);
 }
 
 __global__ __launch_bounds__(kUpdateThreads) void k_bin_update(Parts p, Topo t, const DevClass* classes,

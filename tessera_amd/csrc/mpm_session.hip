@@ -1097,8 +1097,9 @@ BlockLists block_lists(const tmpm_session* s, int set) {
 tmpm_status alloc_topology(tmpm_session* s, uint32_t pblock_cap, uint32_t grid_cap) {
   pblock_cap = std::min(pblock_cap, grid_cap);  // a particle block's grid slot is its id
   // Listed substeps keep the blocks that particles have left until the next
-  // full binning: memory beyond the capacities, so that those cannot make a
-  // scene fail that a full binning of every substep would fit.
+  // full binning: memory beyond the capacities for those.  A scene that visits
+  // more blocks than fit has them made anew on the device (rebuild_lists), so
+  // that none fails that a full binning of every substep would fit.
   const uint32_t ncap = std::max<uint32_t>(s->cap, 1);
   const uint32_t grid_room = grid_cap + grid_cap / 2;
   const uint32_t pblock_room =

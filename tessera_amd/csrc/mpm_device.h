@@ -42,6 +42,7 @@ enum Counter : uint32_t {
   CNT_COUNT = 8,
   // in a cache line of its own: G2P counts here while every workgroup reads the line above
   CNT_STRAYS = 32,          // entries of Topo::stray
+  CNT_STRAYS_ALL = 33,      // of all listed substeps since the last full binning
   CNT_WORDS = 64            // words of the counter array
 };
 // error bits in counters[CNT_ERROR]
@@ -249,7 +250,8 @@ struct Topo {
   // pslot), or kInvalid where its block is to be looked up, and maybe made.
   uint2* stray;
   // pinned host memory (or null): particle and grid blocks of the last full
-  // binning, which the host's next launch shapes follow without waiting
+  // binning, which the host's next launch shapes follow without waiting, and
+  // CNT_STRAYS_ALL, by which it leaves the lists
   uint32_t* seen;
 };
 

@@ -635,7 +635,7 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_offsets(Parts p, Topo t, co
     t.counters[CNT_PARTICLE_BLOCKS] = npb;
     t.counters[CNT_GRID_BLOCKS] = min(npb + total[1], t.grid_cap);
     t.counters[CNT_BINNED] = total[2];
-    t.counters[CNT_STRAYS] = 0;
+    t.counters[CNT_STRAYS] = t.counters[CNT_STRAYS_ALL] = 0;
   }
 }
 
@@ -709,8 +709,8 @@ __global__ __launch_bounds__(256) void k_bin_scatter(Parts p, Topo t) {
 //
 // In a kernel trace the four binning kernels took 39 us of a substep of 153 us
 // at 1M particles, 96 of 576 us at 4M and 19 of 52 us at 8k; this launch takes
-// 5 us without strays and 9 to 15 with some, and writing the lists 4 us of G2P at
-// 1M.
+// 5 us without strays, 9 to 15 with some and about 0.1 us for each of many (the
+// host leaves the lists then), and writing the lists 4 us of G2P at 1M.
 constexpr int kUpdateThreads = 512;
 constexpr uint32_t kClaimed = kInvalid - 1;  // bucket_pblock of a block whose id is being taken
 
@@ -830,6 +830,8 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
     t.counters[CNT_GRID_BLOCKS] = min(npb + s_tiles, t.grid_room);
     t.counters[CNT_BINNED] = binned;
     t.counters[CNT_STRAYS] = 0;
+    t.counters[CNT_STRAYS_ALL] = kInvalid;  // lists do not suit the scene
+    if (t.seen) t.seen[2] = kInvalid;
   }
 }
 
@@ -849,7 +851,7 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
       if (t.scene_err[s] != 0u) t.scene_err[s] |= ERR_STOPPED;
   if (strays == 0) return false;
   const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS], ng = t.counters[CNT_GRID_BLOCKS],
-                 binned = t.counters[CNT_BINNED];
+                 binned = t.counters[CNT_BINNED], all = t.counters[CNT_STRAYS_ALL];
   if (tid == 0) s_new = s_slots = s_rest = s_over = 0;
   __syncthreads();
   // No room: what is left of the phases is skipped (inserts beyond it would fill
@@ -957,6 +959,9 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
     t.counters[CNT_PARTICLE_BLOCKS] = npb + made;
     t.counters[CNT_GRID_BLOCKS] = ng + s_slots;
     t.counters[CNT_STRAYS] = 0;
+    const uint32_t sum = all + min(strays, kInvalid - all);
+    t.counters[CNT_STRAYS_ALL] = sum;
+    if (t.seen) t.seen[2] = sum;
   }
   return false;
 }

@@ -603,12 +603,12 @@ struct tmpm_session {
   std::vector<HostWorld> spare_worlds;  // emptied worlds of retired scenes, reused
   uint32_t force_cap = 0;
   uint32_t last_pblocks = 0, last_gblocks = 0;  // block counts of the last synchronized substep
-  uint32_t* seen = nullptr;                     // Topo::seen: those of the last full binning, 0 for none since
+  uint32_t* seen = nullptr;                     // Topo::seen: of the last full binning and its lists, 0 for none since
   ~tmpm_session() {
     if (seen) (void)hipHostFree(seen);
   }
   void forget_seen() {
-    if (seen) seen[0] = seen[1] = 0;
+    if (seen) seen[0] = seen[1] = seen[2] = 0;
   }
   // Blocks to launch for: a session may run for long without a synchronize, and
   // a spreading scene leaves the count it began with (sand, 79,507 particles from
@@ -644,6 +644,8 @@ struct tmpm_session {
   bool lists_valid = false;  // the last substep left the next one's block lists and the block table
   bool rigid_pending = false;  // within a submission: the next substep runs the last one's rigid step
   int list_read = 0;         // the set the next listed substep reads
+  bool lists_paused = false;  // too many strays: full binnings for list_rest more reorder intervals
+  uint32_t list_rest = 0, list_backoff = 1;
   Topo topo{};
   uint32_t p2g_blocks = 4096, threads_pblock = 64, p2g_threads = 64;
   bool p2g_shape_fixed = false;  // P2G shape set by the tuner or an override, not by scene size
@@ -1185,7 +1187,7 @@ tmpm_status alloc_topology(tmpm_session* s, uint32_t pblock_cap, uint32_t grid_c
   t.node_mask = s->node_mask.as<uint32_t>();
   if (!s->seen) {
     void* q = nullptr;
-    if (hipHostMalloc(&q, 2 * sizeof(uint32_t), hipHostMallocDefault) == hipSuccess) s->seen = static_cast<uint32_t*>(q);
+    if (hipHostMalloc(&q, 3 * sizeof(uint32_t), hipHostMallocDefault) == hipSuccess) s->seen = static_cast<uint32_t*>(q);
     else (void)hipGetLastError();  // launches then follow the synchronized counts only
     s->forget_seen();
   }
@@ -1746,6 +1748,8 @@ tmpm_status prepare_packed(tmpm_session* s, PackedParticles& pk) {
   st = alloc_topology(s, (uint32_t)pcap, (uint32_t)gcap);
   if (st != TMPM_OK) return st;
   s->substeps_since_reorder = 1u << 30;
+  s->lists_paused = false;
+  s->list_backoff = 1;
   s->compacted_last = false;
   s->prepared = true;
   return TMPM_OK;
@@ -1992,6 +1996,32 @@ void effective_p2g_shape(const tmpm_session* s, uint32_t& threads, int& copies) 
 // Where lists are lost, the next substep bins fully and reorders, unless the
 // reorder interval is beyond the span (then only its own reorders happen).
 constexpr uint32_t kListSpan = 32;
+// k_bin_update is one workgroup, about 0.1 us for each particle whose block it
+// has to make: for many of them the four binning kernels of the whole chip are
+// faster.  Thin clouds in flight (us a substep, listed / fully binned): 8,000
+// particles with 310 strays a substep 90 / 128; 30,000 with 440 180 / 192, with
+// 1,100 250 / 205; 100,000 with 310 458 / 466, with 1,340 580 / 485; 400,000 with
+// 11,000 2,900 / 1,810; 1M particles in blocks of 64, about 800, 395 / 379.  The
+// line is on their sum over the listed substeps between two reorders: bodies
+// that cross block faces as a whole stray all at once, and rarely.  Beyond it
+// substeps bin fully for a reorder interval, and for twice as many each time
+// that the lists are tried again and are no better.  The count is the device's:
+// substeps that are under way when the host first sees it are not changed.
+constexpr uint32_t kStraysMost = 600;  // a substep
+constexpr uint32_t kListRestMost = 64;
+void watch_strays(tmpm_session* s, bool synchronized) {
+  if (!s->seen || s->lists_paused) return;
+  const uint32_t span = std::min(s->reorder_interval, kListSpan) - 1;
+  if (((const volatile uint32_t*)s->seen)[2] <= kStraysMost * span) {
+    if (synchronized && s->lists_valid) s->list_backoff = 1;
+    return;
+  }
+  s->seen[2] = 0;
+  s->lists_valid = false;
+  s->lists_paused = true;
+  s->list_rest = s->list_backoff;
+  s->list_backoff = std::min(2 * s->list_backoff, kListRestMost);
+}
 // The most obstacles or bodies for k_rigid_step's one workgroup: with 3 obstacles
 // 4.4 us against 9.6 of the three kernels it replaces (and two launches less),
 // with 504 53 against 58, with 1,024 68 against 58.
@@ -2001,8 +2031,18 @@ SubstepPlan plan_substep(tmpm_session* s, bool apply_force, bool first, bool mor
   SubstepPlan pl;
   std::memset(&pl, 0, sizeof pl);
   pl.p = s->parts(s->cur);
-  const bool may_list = !s->cpic;
-  pl.reorder = s->substeps_since_reorder >= s->reorder_interval ||
+  const bool scheduled = s->substeps_since_reorder >= s->reorder_interval;
+  watch_strays(s, false);
+  if (scheduled && s->lists_paused) {
+    if (s->list_rest > 0) {
+      --s->list_rest;
+    } else {
+      s->lists_paused = false;
+      if (s->seen) s->seen[2] = 0;  // a count from before the pause
+    }
+  }
+  const bool may_list = !s->cpic && !s->lists_paused;
+  pl.reorder = scheduled ||
                (may_list && !s->lists_valid && s->reorder_interval > 1 && s->reorder_interval <= kListSpan);
   if (pl.reorder) pl.q = s->parts(1 - s->cur);
   pl.t = s->topo;
@@ -3289,6 +3329,7 @@ tmpm_status tmpm_session_synchronize(tmpm_session* s) {
       const uint32_t global = s->batch ? (counters[CNT_ERROR] & (ERR_TOPOLOGY | ERR_INTERNAL)) : counters[CNT_ERROR];
       tmpm_status st = status_from_error_bits(global);
       if (st != TMPM_OK) return st;
+      watch_strays(s, true);
       s->forget_seen();
       s->last_pblocks = counters[CNT_PARTICLE_BLOCKS];
       s->last_gblocks = counters[CNT_GRID_BLOCKS];

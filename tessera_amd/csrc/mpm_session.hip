@@ -644,6 +644,13 @@ struct tmpm_session {
   bool lists_valid = false;  // the last substep left the next one's block lists and the block table
   bool rigid_pending = false;  // within a submission: the next substep runs the last one's rigid step
   int list_read = 0;         // the set the next listed substep reads
+  // An edit took the lists away since the last substep; and whether none did
+  // between the last reorder and the substep after it.
+  bool lists_dropped = false, lists_last = true;
+  void drop_lists() {
+    lists_valid = false;
+    lists_dropped = true;
+  }
   bool lists_paused = false;  // too many strays: full binnings for list_rest more reorder intervals
   uint32_t list_rest = 0, list_backoff = 1;
   Topo topo{};
@@ -1132,7 +1139,7 @@ tmpm_status alloc_topology(tmpm_session* s, uint32_t pblock_cap, uint32_t grid_c
   t.stray = s->stray.as<uint2>();
   t.grid_room = grid_room;
   t.pblock_room = pblock_room;
-  s->lists_valid = false;
+  s->drop_lists();
   s->topo_cap = s->cap;
   HIP_TRY(s->pslot.alloc(4ull * std::max<uint32_t>(s->cap, 1)));
   HIP_TRY(s->prank.alloc(4ull * std::max<uint32_t>(s->cap, 1)));
@@ -1675,7 +1682,7 @@ tmpm_status prepare(tmpm_session* s) {
 tmpm_status prepare_packed(tmpm_session* s, PackedParticles& pk) {
   s->prepared = false;
   s->topo_valid = false;
-  s->lists_valid = false;
+  s->drop_lists();
   if (s->scenes.size() > 0xffffu) return fail(TMPM_CAPACITY, "too many scenes");
   uint64_t total = 0;
   for (auto& scene : s->scenes) {
@@ -1761,7 +1768,7 @@ hipError_t enqueue_binning(tmpm_session* s, const Parts& p) {
   const DevScene* sc = s->scene_plain.as<DevScene>();
   Topo& t = s->topo;
   hipError_t e;
-  s->lists_valid = false;  // the table and the blocks' ranges are made anew
+  s->drop_lists();  // the table and the blocks' ranges are made anew
   if (s->table_dirty) {
     if ((e = timed(s, "k_topo_clear", [&] { launch_topo_clear(t, s->stream); })) != hipSuccess) return e;
     s->table_dirty = false;
@@ -1994,7 +2001,15 @@ void effective_p2g_shape(const tmpm_session* s, uint32_t& threads, int& copies) 
 // since the reorder, so that lists stay short.  With CPIC a particle changes
 // its block key without moving to another cell: every substep bins fully.
 // Where lists are lost, the next substep bins fully and reorders, unless the
-// reorder interval is beyond the span (then only its own reorders happen).
+// reorder interval is beyond the span (then only its own reorders happen).  A
+// reorder writes lists, and is brought forward for them, only if a substep is
+// going to use them as far as the host can tell: another one of this
+// submission, or as after the last reorder.  Edits before every single substep
+// would otherwise have lists written and the block table cleared by a launch of
+// its own each time.  A batch of 16 scenes of 60,000, a submission of one substep
+// after each admission: 231 us with lists written each time, 194 now; 201 and 200
+// where a scene is removed too (that reorders anyway).  Before every second
+// substep 162 both ways, and 169 without lists.
 constexpr uint32_t kListSpan = 32;
 // k_bin_update is one workgroup, about 0.1 us for each particle whose block it
 // has to make: for many of them the four binning kernels of the whole chip are
@@ -2042,13 +2057,15 @@ SubstepPlan plan_substep(tmpm_session* s, bool apply_force, bool first, bool mor
     }
   }
   const bool may_list = !s->cpic && !s->lists_paused;
+  if (s->compacted_last) s->lists_last = !s->lists_dropped;  // the last substep reordered
+  const bool use = more || s->lists_last;
   pl.reorder = scheduled ||
-               (may_list && !s->lists_valid && s->reorder_interval > 1 && s->reorder_interval <= kListSpan);
+               (may_list && !s->lists_valid && use && s->reorder_interval > 1 && s->reorder_interval <= kListSpan);
   if (pl.reorder) pl.q = s->parts(1 - s->cur);
   pl.t = s->topo;
   const bool listed = !pl.reorder && may_list && s->lists_valid;
   const uint32_t since = pl.reorder ? 1u : s->substeps_since_reorder + 1;  // after this substep
-  const bool build = may_list && (pl.reorder || listed) && since < s->reorder_interval && since < kListSpan;
+  const bool build = may_list && ((pl.reorder && use) || listed) && since < s->reorder_interval && since < kListSpan;
   pl.t.listed = listed ? 1 : 0;
   pl.t.build = build ? 1 : 0;
   const int read = listed ? s->list_read : 0;
@@ -2215,6 +2232,7 @@ hipError_t enqueue_substep(tmpm_session* s, bool apply_force, bool first, bool m
   const hipError_t e = s->use_graphs && !s->timing && !pl.audit ? launch_graph(s, pl) : launch_plan(s, pl);
   if (e != hipSuccess) return e;
   s->lists_valid = pl.t.build != 0;
+  s->lists_dropped = false;
   s->rigid_pending = pl.rigid_next && !pl.rigid_step;
   s->list_read = pl.t.listed ? 1 - s->list_read : 1;
   s->table_dirty = pl.t.build != 0;  // otherwise G2P cleared the block table
@@ -3157,7 +3175,7 @@ tmpm_status commit_staged(tmpm_session* s, tmpm_staged_scene& staged, uint32_t* 
     swap_bufs(s->synced, synced);
     s->cap = cap;
   }
-  s->lists_valid = false;  // the new particles are on no list
+  s->drop_lists();  // the new particles are on no list
   if ((st = upload_particles(s, pk, s->n)) != TMPM_OK) return broken(st);
   s->n += (uint32_t)pk.size();
   s->n_enabled = s->n;
@@ -3406,7 +3424,7 @@ tmpm_status tmpm_session_synchronize(tmpm_session* s) {
         scene.status = status_from_error_bits(scene_bits[k]);  // the last synchronized world stays readable
         stopped = true;
         if (s->prepared && scene.count) {
-          s->lists_valid = false;  // its particles leave their blocks' ranges and lists
+          s->drop_lists();  // its particles leave their blocks' ranges and lists
           launch_retire(s->parts(s->cur), scene.first, scene.count, s->stream);
           HIP_TRY(hipGetLastError());
         }
@@ -3786,7 +3804,7 @@ tmpm_status tmpm_batch_remove_scene(tmpm_session* s, uint32_t scene) {
       // next reorder drops them) and the insertion indices above its range
       // close the gap, here and in the synchronized copy.
       Parts p = s->parts(s->cur);
-      s->lists_valid = false;
+      s->drop_lists();
       launch_retire(p, first, count, s->stream);
       launch_renumber(p.ins_id, s->n, first, count, s->stream);
       launch_renumber(s->synced.ins_id.as<uint32_t>(), s->synced_n, first, count, s->stream);

@@ -37,6 +37,7 @@
 
 #include "mpm_device.h"
 #include "mpm_kernels.h"
+#include "mpm_root.h"
 
 namespace tmpm {
 
@@ -3038,18 +3039,15 @@ __global__ __launch_bounds__(256) void k_live_count(Topo t) {
 // candidate lies on the surface, or the mesh's scale over- or underflows), the
 // candidate is left to k_mesh_inside, one thread per candidate that sums the
 // angles in the reference's order.
-// Bound by f64 issue (75 f64 operations per pair, ~50 us of it on all CUs).
+// Bound by f64 issue (81 f64 operations per pair, ~55 us of it on all CUs).
 // 1,280 triangles and 18,400 candidates: 84 us, and 4 us for k_mesh_inside over
 // the undecided ones; 137 us with each group's triangles in one workgroup; 704 us
 // with an atan2 per pair on one thread per candidate (72 workgroups).
 // ---------------------------------------------------------------------------
 constexpr uint8_t kMeshUndecided = 2;
 
-// sqrt(x) to ~1e-15 for normal x > 0; NaN at 0
-__device__ __forceinline__ double mesh_root(double x) {
-  const double y = __builtin_amdgcn_rsq(x), r = x * y;
-  return __builtin_fma(0.5 * y, __builtin_fma(-r, r, x), r);
-}
+// sqrt(x) for normal x > 0; NaN at 0
+__device__ __forceinline__ double mesh_root(double x) { return refine_root(x, __builtin_amdgcn_rsq(x)); }
 
 // From the whole sum (NaN: undecided): a turn and more, none, or in between.
 __device__ __forceinline__ uint8_t mesh_decide(double angle) {

@@ -51,7 +51,7 @@ enum ErrorBit : uint32_t {
   ERR_TOPOLOGY = 2u,        // hash or grid capacity exhausted: Capacity
   ERR_FIXED_RANGE = 4u,     // fixed-point contribution out of range: Capacity
   ERR_INTERNAL = 8u,        // inconsistent binning (must never happen)
-  ERR_STOPPED = 16u         // scene_err of a batch only: had failed before the listed substep at hand
+  ERR_STOPPED = 16u         // scene_err of a batch only: its lists have been emptied
 };
 
 // Device material codes.  Snow and sand use the corotated stress, sand-NH the
@@ -213,8 +213,8 @@ struct Topo {
   uint32_t* sorted;         // binned order -> particle storage index
   uint32_t* counters;
   uint32_t* scene_err;      // per scene: error bits of its particles and blocks
-  uint32_t isolate;         // batches: binning skips the particles of scenes whose error bits are set
-  uint32_t scene_total;     // entries of scene_err in use
+  // batches: the scenes (else 0); binning skips the particles of those whose error bits are set
+  uint32_t isolate;
   // binning lists: insert workgroup g bins particles [g * bin_span, (g + 1) * bin_span)
   uint32_t bin_span;        // particles per binning workgroup (multiple of 256)
   uint32_t bin_groups;      // binning workgroups

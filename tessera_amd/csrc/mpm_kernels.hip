@@ -736,6 +736,7 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
   if (tid == 0) s_blocks = s_tiles = 0;
   bool over = false;
   phase_end();
+#pragma unroll 1
   for (uint32_t b = tid; b <= t.bucket_mask; b += kUpdateThreads) {
     t.owner[b] = 0;
     t.bucket_count[b] = 0;
@@ -743,6 +744,7 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
     t.bucket_pblock[b] = t.bucket_slot[b] = kInvalid;
   }
   phase_end();
+#pragma unroll 1
   for (uint32_t i = tid; i < p.n; i += kUpdateThreads) {
     const float4 pm = p.pos_mass[i];
     const DevClass& c = classes[p.cls[i]];
@@ -750,8 +752,8 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
     int3 cell;
     if (pm.w > 0.0f && !(t.isolate && t.scene_err[c.region >> 16] != 0u) && cell3(pm, c.inv_h, cell)) {
       bool claimed;
-      const int4 key = make_int4(cell.x >> 2, cell.y >> 2, cell.z >> 2, (int)c.region);
-      b = hash_insert(p, t, classes, scenes, key, i + 1, claimed);
+      b = hash_insert<false, true>(p, t, classes, scenes,
+                                   make_int4(cell.x >> 2, cell.y >> 2, cell.z >> 2, (int)c.region), i + 1, claimed);
       if (b == kInvalid) {
         over = true;
       } else {
@@ -761,7 +763,7 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
           if (k < room) {
             t.pblock_nbr[8 * k] = b;
             t.bucket_pblock[b] = t.bucket_slot[b] = k;
-            t.grid_key[k] = key;
+            t.grid_key[k] = t.bkey[b];
             clear_rev(t, k);
           } else {
             over = true;
@@ -773,6 +775,7 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
   }
   phase_end();
   const uint32_t npb = min(s_blocks, room);
+#pragma unroll 1
   for (uint32_t q = tid; q < 7 * npb; q += kUpdateThreads) {
     const uint32_t k = q / 7u, d = q % 7u + 1u, b = t.pblock_nbr[8 * k];
     int4 key = t.grid_key[k];
@@ -787,7 +790,7 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
       const uint32_t slot = npb + atomicAdd(&s_tiles, 1u);
       if (slot < t.grid_room) {
         t.bucket_slot[got] = slot;
-        t.grid_key[slot] = key;
+        t.grid_key[slot] = t.bkey[got];
         clear_rev(t, slot);
       } else {
         over = true;
@@ -796,6 +799,7 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
     t.pblock_nbr[8 * k + d] = got;
   }
   phase_end();
+#pragma unroll 1
   for (uint32_t q = tid; q < 8 * npb; q += kUpdateThreads) {
     const uint32_t b = t.pblock_nbr[q], slot = b == kInvalid ? kInvalid : t.bucket_slot[b];
     t.pblock_slot8[q] = slot;
@@ -805,14 +809,17 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
   const uint32_t run = (npb + kUpdateThreads - 1) / kUpdateThreads;
   const uint32_t k0 = min(tid * run, npb), k1 = min(k0 + run, npb);
   uint32_t sum = 0;
+#pragma unroll 1
   for (uint32_t k = k0; k < k1; ++k) sum += t.bucket_count[t.pblock_nbr[8 * k]];
   s_sum[tid] = sum;
   phase_end();
   uint32_t at = 0, binned = 0;
+#pragma unroll 1
   for (uint32_t u = 0; u < kUpdateThreads; ++u) {
     if (u < tid) at += s_sum[u];
     binned += s_sum[u];
   }
+#pragma unroll 1
   for (uint32_t k = k0; k < k1; ++k) {
     const uint32_t len = t.bucket_count[t.pblock_nbr[8 * k]];
     t.pblock_start[k] = at;
@@ -821,6 +828,7 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
     at += len;
   }
   phase_end();
+#pragma unroll 1
   for (uint32_t i = tid; i < p.n; i += kUpdateThreads) {
     const uint32_t b = t.pslot[i], k = b == kInvalid ? kInvalid : t.bucket_pblock[b];
     if (k != kInvalid) t.cur.idx[t.pblock_start[k] + (uint64_t)t.cur.pitch * k + t.prank[i]] = i;
@@ -843,16 +851,9 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
   __shared__ uint32_t s_new, s_slots, s_rest, s_over;
   const uint32_t strays = min(t.counters[CNT_STRAYS], p.n);
   const uint32_t tid = threadIdx.x;
-  // A batch scene that failed in an earlier substep is not binned any more
-  // (see k_bin_insert); on the lists its particles still are, so P2G drops
-  // those of the scenes marked here.  Scenes that fail in this substep's P2G
-  // are not marked: they run it to its end, as after a full binning.
-  if (t.isolate && (t.counters[CNT_ERROR] & (ERR_RESIDENT | ERR_FIXED_RANGE)) != 0u)
-    for (uint32_t s = tid; s < t.scene_total; s += kUpdateThreads)
-      if (t.scene_err[s] != 0u) t.scene_err[s] |= ERR_STOPPED;
   if (strays == 0) return false;
   const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS], ng = t.counters[CNT_GRID_BLOCKS],
-                 binned = t.counters[CNT_BINNED], all = t.counters[CNT_STRAYS_ALL];
+                 binned = t.counters[CNT_BINNED];
   if (tid == 0) s_new = s_slots = s_rest = s_over = 0;
   __syncthreads();
   // No room: what is left of the phases is skipped (inserts beyond it would fill
@@ -861,12 +862,12 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
   auto no_room = [&] { over = *(volatile uint32_t*)&s_over != 0u || over; return over; };
   auto overflow = [&] { over = true; *(volatile uint32_t*)&s_over = 1u; };
   // grid slot of a new bucket
-  auto take_slot = [&](uint32_t b, int4 key) {
+  auto take_slot = [&](uint32_t b) {
     const uint32_t slot = ng + atomicAdd(&s_slots, 1u);
     t.bucket_pblock[b] = t.bucket_slot[b] = kInvalid;
     if (slot >= t.grid_room) return overflow();
     t.bucket_slot[b] = slot;
-    t.grid_key[slot] = key;
+    t.grid_key[slot] = t.bkey[b];
     clear_rev(t, slot);
   };
   // the buckets of the particles whose block is to be looked up (pslot: kInvalid for none)
@@ -880,10 +881,10 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
     int3 cell;
     if (!no_room() && !(t.isolate && t.scene_err[c.region >> 16] != 0u) && cell3(p.pos_mass[i], c.inv_h, cell)) {
       bool claimed;
-      const int4 key = make_int4(cell.x >> 2, cell.y >> 2, cell.z >> 2, (int)c.region);
-      b = hash_insert<false, true>(p, t, classes, scenes, key, i + 1, claimed);
+      b = hash_insert<false, true>(p, t, classes, scenes,
+                                   make_int4(cell.x >> 2, cell.y >> 2, cell.z >> 2, (int)c.region), i + 1, claimed);
       if (b == kInvalid) overflow();
-      else if (claimed) take_slot(b, key);
+      else if (claimed) take_slot(b);
     }
     t.pslot[i] = b;
   }
@@ -917,7 +918,7 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
     const uint32_t got =
         no_room() ? kInvalid : hash_insert<false, true>(p, t, classes, scenes, k, p.n + 1 + 8 * b + d, claimed);
     if (got == kInvalid) overflow();
-    else if (claimed) take_slot(got, k);
+    else if (claimed) take_slot(got);
     t.pblock_nbr[8 * pb + d] = got;
   }
   if (__syncthreads_or(over)) return true;
@@ -960,7 +961,7 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
     t.counters[CNT_PARTICLE_BLOCKS] = npb + made;
     t.counters[CNT_GRID_BLOCKS] = ng + s_slots;
     t.counters[CNT_STRAYS] = 0;
-    const uint32_t sum = all + min(strays, kInvalid - all);
+    const uint32_t all = t.counters[CNT_STRAYS_ALL], sum = all + min(strays, kInvalid - all);
     t.counters[CNT_STRAYS_ALL] = sum;
     if (t.seen) t.seen[2] = sum;
   }
@@ -970,9 +971,33 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
 __device__ __forceinline__ void update_lists(const Parts& p, const Topo& t, const DevClass* classes,
                                              const DevScene* scenes) {
   if (extend_lists(p, t, classes, scenes)) rebuild_lists(p, t, classes, scenes);
+  // A batch scene that failed in an earlier substep is not binned any more (see
+  // k_bin_insert); on the lists its particles still are, so the lists of its
+  // blocks are emptied, once: they stay empty.
+  if (!t.isolate || (t.counters[CNT_ERROR] & (ERR_RESIDENT | ERR_FIXED_RANGE)) == 0u) return;
+  bool failed = false;
+#pragma unroll 1
+  for (uint32_t s = threadIdx.x; s < t.isolate; s += kUpdateThreads)
+    if (t.scene_err[s] != 0u && (t.scene_err[s] & ERR_STOPPED) == 0u) {
+      t.scene_err[s] |= ERR_STOPPED;
+      failed = true;
+    }
+  if (!__syncthreads_or(failed)) return;
+  phase_end();
+  const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS];
+#pragma unroll 1
+  for (uint32_t k = threadIdx.x; k < npb; k += kUpdateThreads) {
+    const uint32_t own = t.pblock_slot8[8 * k];
+    if (own != kInvalid && t.scene_err[(uint32_t)t.grid_key[own].w >> 16] != 0u) t.cur.meta[k] = make_uint4(0, 0, 0, 0);
+  }
 }
 
-__global__ __launch_bounds__(kUpdateThreads) void k_bin_update(Parts p, Topo t, const DevClass* classes,
+// At most 32 VGPRs (the attribute counts half of CDNA's unified file): the
+// workgroup is then resident beside two wavefronts per SIMD of another session's
+// plastic G2P, which leave 64.  With 40 it waited for them: three sessions of
+// 79,507 sand particles at a time, 25.2 us a substep each against 24.4; with 256
+// threads and 40 as fast there, but 50% slower over hundreds of strays.
+__global__ __launch_bounds__(kUpdateThreads) __attribute__((amdgpu_num_vgpr(16))) void k_bin_update(Parts p, Topo t, const DevClass* classes,
                                                                const DevScene* scenes) {
   update_lists(p, t, classes, scenes);
 }
@@ -1993,18 +2018,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS
     }
     const int4 key = uniform4(t.grid_key[own]);
     const DevScene& sc = scenes[(uint32_t)key.w >> 16];
-    // A scene that k_bin_update found failed: the block takes part in nothing
-    // more in this substep, here and in G2P (which finds its list empty).
-    const bool stopped =
-        t.listed && t.isolate && (uniform1(t.scene_err[(uint32_t)key.w >> 16]) & ERR_STOPPED) != 0u;
-    const uint32_t todo = stopped ? 0u : total;
-    if (stopped && tid == 0) t.cur.meta[k] = make_uint4(0, 0, 0, 0);
     const float h = sc.h, inv_h = sc.inv_h;
     const float stress_scale = -sc.dt * sc.inv_d;
     const float mscale = exp2f((float)sc.mass_shift), pscale = exp2f((float)sc.mom_shift);
     const int ox = key.x * kBlockCells, oy = key.y * kBlockCells, oz = key.z * kBlockCells;
-    bool bad = false, range = !stopped && total - list.holes > kP2GMaxBlock;
-    for (uint32_t j = tid; j < todo; j += THREADS) {
+    bool bad = false, range = total - list.holes > kP2GMaxBlock;
+    for (uint32_t j = tid; j < total; j += THREADS) {
       const uint32_t i = j == (uint32_t)tid               ? i_first
                          : j == (uint32_t)(tid + THREADS) ? i_second
                                                           : block_particle(list, j);

@@ -1019,8 +1019,7 @@ tmpm_status upload_scene(tmpm_session* s) {
   HIP_TRY(hipMemcpy(s->scene_plain.ptr, plain.data(), sizeof(DevScene) * n, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(s->scene_force.ptr, forced.data(), sizeof(DevScene) * n, hipMemcpyHostToDevice));
   s->topo.scene_err = s->scene_err.as<uint32_t>();
-  s->topo.isolate = s->batch ? 1u : 0u;
-  s->topo.scene_total = (uint32_t)n;
+  s->topo.isolate = s->batch ? (uint32_t)n : 0u;
   return TMPM_OK;
 }
 

@@ -455,7 +455,12 @@ tmpm_status tmpm_session_autotune(tmpm_session* s, uint32_t trial, uint32_t* sub
  * wider workgroups, so that a launch still fills the chip: P2G 128 threads;
  * G2P 128 threads below 8,192 blocks or from 192 particles per block, 256
  * below 4,096 blocks or from 288 particles per block.  P2G uses one tile
- * copy unless tuned to two. */
+ * copy unless tuned to two.  The widest of these, by size or tuned, stand for
+ * workgroups that widen as the blocks get few: P2G's 128 threads with one copy
+ * launch as 256 up to 1,024 blocks and 512 up to 512, G2P's 256 as 512 up to 512
+ * blocks without plastic materials and obstacle shapes.  A width that
+ * TMPM_P2G_THREADS (64, 128, 256, 512) or TMPM_PBLOCK_THREADS (64, 128, 192, 256,
+ * 512) sets in the environment launches as reported. */
 tmpm_status tmpm_session_launch_config(tmpm_session* s, int32_t out[5]);
 tmpm_status tmpm_session_kernel_times(tmpm_session* s, char* names_csv, uint64_t names_cap, double* avg_ms,
                                       uint64_t* calls, uint32_t cap, uint32_t* count_out);

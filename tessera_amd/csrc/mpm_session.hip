@@ -657,6 +657,7 @@ struct tmpm_session {
   uint32_t p2g_blocks = 4096, threads_pblock = 64, p2g_threads = 64;
   bool p2g_shape_fixed = false;  // P2G shape set by the tuner or an override, not by scene size
   bool g2p_shape_fixed = false;  // likewise for the G2P workgroup size
+  bool p2g_exact = false, g2p_exact = false;  // set by an override: runs as it is, also on few blocks
   int p2g_copies = 1;
   bool topo_valid = false;  // topology arrays describe the current device state
   bool table_dirty = true;  // block hash needs clearing before the next binning
@@ -1073,21 +1074,23 @@ tmpm_status build_scene(SceneState& scene) {
   return TMPM_OK;
 }
 
-// Launch-shape overrides for tuning sweeps, read once per session.
+// Launch-shape overrides for tuning sweeps, read once per session.  They run as
+// given (P2G's 256 and 512 with one tile copy, G2P's 512 in sessions without
+// plastic materials and obstacle shapes).
 void read_tuning_env(tmpm_session* s) {
   if (const char* v = std::getenv("TMPM_PBLOCK_THREADS")) {
     int th = std::atoi(v);
-    if (th == 64 || th == 128 || th == 192 || th == 256) s->threads_pblock = (uint32_t)th;
-    s->g2p_shape_fixed = true;
+    if (th == 64 || th == 128 || th == 192 || th == 256 || th == 512) s->threads_pblock = (uint32_t)th;
+    s->g2p_shape_fixed = s->g2p_exact = true;
   }
   if (const char* v = std::getenv("TMPM_P2G_THREADS")) {
     int th = std::atoi(v);
-    if (th == 64 || th == 128) s->p2g_threads = (uint32_t)th;
-    s->p2g_shape_fixed = true;
+    if (th == 64 || th == 128 || th == 256 || th == 512) s->p2g_threads = (uint32_t)th;
+    s->p2g_shape_fixed = s->p2g_exact = true;
   }
   if (const char* v = std::getenv("TMPM_P2G_COPIES")) {
     s->p2g_copies = std::atoi(v) == 1 ? 1 : 2;
-    s->p2g_shape_fixed = true;
+    s->p2g_shape_fixed = s->p2g_exact = true;
   }
   if (const char* v = std::getenv("TMPM_GRAPHS")) s->use_graphs = std::atoi(v) != 0;
   if (const char* v = std::getenv("TMPM_REORDER_INTERVAL")) {
@@ -1838,8 +1841,8 @@ uint32_t particles_per_block(const tmpm_session* s) {
   return s->last_pblocks ? (uint32_t)(s->n / s->last_pblocks) : 0u;
 }
 
-// The launch of a shape's widest workgroups (P2G's 128 threads, G2P's 256) goes
-// wider yet while the chip has room for all blocks at once: 16 wavefronts per
+// The launch of a shape's widest workgroups (P2G's 128 threads, G2P's 256), by
+// size or as the tuner found it, not by an override, goes wider yet while the chip has room for all blocks at once: 16 wavefronts per
 // CU of P2G and 20 of the plain G2P are resident, so two workgroups of 512
 // threads each, or four of 256.  A few blocks are then as fast as their longest
 // chain: the passes over the particles, P2G's flush and the tile loads, all
@@ -1854,11 +1857,11 @@ uint32_t particles_per_block(const tmpm_session* s) {
 //         10.6 / 15.4;  900 of 278: 43.8 / 29.7 / 20.3 / 22.6.
 uint32_t widened_p2g(const tmpm_session* s, uint32_t threads, int copies) {
   const uint32_t b = s->pblocks_now();
-  if (threads != 128 || copies != 1 || b > 4 * kCus) return threads;
+  if (s->p2g_exact || threads != 128 || copies != 1 || b > 4 * kCus) return threads;
   return b <= 2 * kCus ? 512u : 256u;
 }
 uint32_t widened_g2p(const tmpm_session* s, uint32_t threads) {
-  return threads == 256 && !s->plastic && !s->shapes && s->pblocks_now() <= 2 * kCus ? 512u : threads;
+  return !s->g2p_exact && threads == 256 && !s->plastic && !s->shapes && s->pblocks_now() <= 2 * kCus ? 512u : threads;
 }
 
 // Workgroups of a launch that takes one block each (every kernel strides over
@@ -1966,7 +1969,7 @@ TuneKey tune_key(const tmpm_session* s) {
 bool cached_shape(const tmpm_session* s, TuneShape& out) { return tune_cache().find(tune_key(s), out); }
 
 uint32_t effective_g2p_threads(const tmpm_session* s) {
-  if (s->g2p_shape_fixed) return s->threads_pblock;
+  if (s->g2p_shape_fixed) return s->plastic || s->shapes ? std::min(s->threads_pblock, 256u) : s->threads_pblock;
   TuneShape c;
   if (cached_shape(s, c)) return c.g2p_threads;
   const uint32_t b = s->last_pblocks, ppb = particles_per_block(s);
@@ -1978,20 +1981,20 @@ uint32_t effective_g2p_threads(const tmpm_session* s) {
 }
 
 void effective_p2g_shape(const tmpm_session* s, uint32_t& threads, int& copies) {
+  TuneShape c;
   if (s->p2g_shape_fixed) {
     threads = s->p2g_threads;
     copies = s->p2g_copies;
-    return;
-  }
-  TuneShape c;
-  if (cached_shape(s, c)) {
+  } else if (cached_shape(s, c)) {
     threads = c.p2g_threads;
     copies = c.p2g_copies;
-    return;
+  } else {
+    threads = s->last_pblocks < kFillBlocks || particles_per_block(s) >= 192 ? 128u : 64u;
+    copies = 1;
   }
-  const uint32_t b = s->last_pblocks;
-  threads = b < kFillBlocks || particles_per_block(s) >= 192 || s->plastic ? 128u : 64u;
-  copies = 1;
+  // the kernels there are (launch_p2g)
+  if (s->plastic) threads = std::max(threads, 128u);
+  if (s->plastic || threads > 128) copies = 1;
 }
 
 // Listed substeps.  A substep after a reorder takes its particles from the
@@ -4153,6 +4156,7 @@ tmpm_status tmpm_session_autotune(tmpm_session* s, uint32_t trial, uint32_t* sub
       s->reorder_interval = hit.reorder_interval;
       s->use_graphs = hit.graphs != 0;
       s->p2g_shape_fixed = s->g2p_shape_fixed = true;
+      s->p2g_exact = s->g2p_exact = false;
       if (!s->use_graphs) destroy_graphs(s);
       return TMPM_OK;
     }
@@ -4217,11 +4221,12 @@ tmpm_status tmpm_session_autotune(tmpm_session* s, uint32_t trial, uint32_t* sub
       return TMPM_OK;
     };
     st = run(std::min<uint32_t>(trial, 16), nullptr);  // warm-up
+    s->p2g_exact = s->g2p_exact = false;  // the tuner's widths are those of many blocks
     if (st == TMPM_OK && !stopped) {
       effective_p2g_shape(s, s->p2g_threads, s->p2g_copies);  // trials start from the shape in use
       s->p2g_shape_fixed = true;  // the trials' shapes, not the size-based default, run from here on
       const int cur = (int)s->p2g_threads * 10 + s->p2g_copies;
-      st = tune({642, 641, 1282, 1281}, [&](int v) { s->p2g_threads = (uint32_t)(v / 10); s->p2g_copies = v % 10; }, cur);
+      if (!s->plastic) st = tune({642, 641, 1282, 1281}, [&](int v) { s->p2g_threads = (uint32_t)(v / 10); s->p2g_copies = v % 10; }, cur);
     }
     if (st == TMPM_OK && !stopped) {
       s->threads_pblock = effective_g2p_threads(s);  // trials start from the size in use

@@ -848,28 +848,15 @@ __device__ __forceinline__ void rebuild_lists(const Parts& p, const Topo& t, con
 // Uniform over the workgroup.
 __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, const DevClass* classes,
                                              const DevScene* scenes) {
-  __shared__ uint32_t s_new, s_slots, s_rest, s_over;
+  __shared__ uint32_t s_new, s_slots, s_rest;
+  __shared__ uint32_t s_over[2];  // no room: found with the particle blocks, with their neighbours
   const uint32_t strays = min(t.counters[CNT_STRAYS], p.n);
   const uint32_t tid = threadIdx.x;
   if (strays == 0) return false;
-  const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS], ng = t.counters[CNT_GRID_BLOCKS],
-                 binned = t.counters[CNT_BINNED];
-  if (tid == 0) s_new = s_slots = s_rest = s_over = 0;
-  __syncthreads();
-  // No room: what is left of the phases is skipped (inserts beyond it would fill
-  // the table, and each then probes all of it).
-  bool over = false;
-  auto no_room = [&] { over = *(volatile uint32_t*)&s_over != 0u || over; return over; };
-  auto overflow = [&] { over = true; *(volatile uint32_t*)&s_over = 1u; };
-  // grid slot of a new bucket
-  auto take_slot = [&](uint32_t b) {
-    const uint32_t slot = ng + atomicAdd(&s_slots, 1u);
-    t.bucket_pblock[b] = t.bucket_slot[b] = kInvalid;
-    if (slot >= t.grid_room) return overflow();
-    t.bucket_slot[b] = slot;
-    t.grid_key[slot] = t.bkey[b];
-    clear_rev(t, slot);
-  };
+  const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS], ng = t.counters[CNT_GRID_BLOCKS];
+  // the table must not fill: each insert would then probe all of it
+  if (ng + strays > t.bucket_mask - (t.bucket_mask >> 3)) return true;
+  if (tid == 0) s_new = s_slots = s_rest = s_over[0] = s_over[1] = 0;
   // the buckets of the particles whose block is to be looked up (pslot: kInvalid for none)
   for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
     const uint2 e = t.stray[s];
@@ -879,16 +866,27 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
     uint32_t b = kInvalid;
     // a failed scene makes no blocks any more, as in k_bin_insert
     int3 cell;
-    if (!no_room() && !(t.isolate && t.scene_err[c.region >> 16] != 0u) && cell3(p.pos_mass[i], c.inv_h, cell)) {
+    if (!(t.isolate && t.scene_err[c.region >> 16] != 0u) && cell3(p.pos_mass[i], c.inv_h, cell)) {
       bool claimed;
       b = hash_insert<false, true>(p, t, classes, scenes,
                                    make_int4(cell.x >> 2, cell.y >> 2, cell.z >> 2, (int)c.region), i + 1, claimed);
-      if (b == kInvalid) overflow();
-      else if (claimed) take_slot(b);
+      if (b == kInvalid) atomicOr(&t.counters[CNT_ERROR], ERR_INTERNAL);  // the table is not full
+      else if (claimed) t.bucket_pblock[b] = t.bucket_slot[b] = kInvalid;
     }
     t.pslot[i] = b;
   }
-  if (__syncthreads_or(over)) return true;
+  __syncthreads();
+  // grid slot of a bucket that has none
+  auto take_slot = [&](uint32_t b, int phase) {
+    const uint32_t slot = ng + atomicAdd(&s_slots, 1u);
+    if (slot >= t.grid_room) {
+      s_over[phase] = 1;
+      return;
+    }
+    t.bucket_slot[b] = slot;
+    t.grid_key[slot] = t.bkey[b];
+    clear_rev(t, slot);
+  };
   // new particle blocks: the first stray of each takes its id
   for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
     const uint2 e = t.stray[s];
@@ -896,16 +894,18 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
     if (b == kInvalid || atomicCAS(&t.bucket_pblock[b], kInvalid, kClaimed) != kInvalid) continue;
     const uint32_t pb = npb + atomicAdd(&s_new, 1u);
     if (pb >= t.pblock_room) {
-      overflow();
+      s_over[0] = 1;
       continue;
     }
+    if (t.bucket_slot[b] == kInvalid) take_slot(b, 0);
     t.pblock_nbr[8 * pb] = b;
-    t.pblock_start[pb] = binned;
+    t.pblock_start[pb] = t.counters[CNT_BINNED];
     t.pblock_len[pb] = 0;
     t.cur.meta[pb] = make_uint4(0, 0, 0, 0);
     t.bucket_pblock[b] = pb;
   }
-  if (__syncthreads_or(over)) return true;
+  __syncthreads();
+  if (s_over[0]) return true;  // not written any more
   const uint32_t made = s_new;
   for (uint32_t q = tid; q < 7 * made; q += kUpdateThreads) {
     const uint32_t pb = npb + q / 7u, d = q % 7u + 1u;
@@ -914,14 +914,19 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
     k.x += (int)(d >> 2);
     k.y += (int)((d >> 1) & 1);
     k.z += (int)(d & 1);
-    bool claimed = false;
-    const uint32_t got =
-        no_room() ? kInvalid : hash_insert<false, true>(p, t, classes, scenes, k, p.n + 1 + 8 * b + d, claimed);
-    if (got == kInvalid) overflow();
-    else if (claimed) take_slot(got);
+    if (*(volatile uint32_t*)&s_over[1] != 0u) break;  // inserts beyond the room would fill the table
+    bool claimed;
+    const uint32_t got = hash_insert<false, true>(p, t, classes, scenes, k, p.n + 1 + 8 * b + d, claimed);
+    if (got == kInvalid) {
+      s_over[1] = 1;
+    } else if (claimed) {
+      t.bucket_pblock[got] = t.bucket_slot[got] = kInvalid;
+      take_slot(got, 1);
+    }
     t.pblock_nbr[8 * pb + d] = got;
   }
-  if (__syncthreads_or(over)) return true;
+  __syncthreads();
+  if (s_over[1]) return true;
   for (uint32_t q = tid; q < 8 * made; q += kUpdateThreads) {
     const uint32_t pb = npb + (q >> 3), d = q & 7, b = t.pblock_nbr[8 * pb + d];
     const uint32_t slot = b == kInvalid ? kInvalid : t.bucket_slot[b];

@@ -854,9 +854,20 @@ __device__ __forceinline__ bool extend_lists(const Parts& p, const Topo& t, cons
   const uint32_t tid = threadIdx.x;
   if (strays == 0) return false;
   const uint32_t npb = t.counters[CNT_PARTICLE_BLOCKS], ng = t.counters[CNT_GRID_BLOCKS];
-  // the table must not fill: each insert would then probe all of it
-  if (ng + strays > t.bucket_mask - (t.bucket_mask >> 3)) return true;
   if (tid == 0) s_new = s_slots = s_rest = s_over[0] = s_over[1] = 0;
+  // the table must not fill: each insert would then probe all of it
+  const uint32_t most = t.bucket_mask - (t.bucket_mask >> 3);
+  if (ng + strays > most) {
+    // those that have a block make no key
+    __syncthreads();
+    for (uint32_t s = tid; s < strays; s += kUpdateThreads)
+      if (t.stray[s].y == kInvalid) atomicAdd(&s_new, 1u);
+    __syncthreads();
+    const bool full = ng + s_new > most;
+    __syncthreads();
+    if (full) return true;
+    if (tid == 0) s_new = 0;
+  }
   // the buckets of the particles whose block is to be looked up (pslot: kInvalid for none)
   for (uint32_t s = tid; s < strays; s += kUpdateThreads) {
     const uint2 e = t.stray[s];

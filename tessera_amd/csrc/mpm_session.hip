@@ -606,6 +606,7 @@ struct tmpm_session {
   uint32_t* seen = nullptr;                     // Topo::seen: of the last full binning and its lists, 0 for none since
   ~tmpm_session() {
     if (seen) (void)hipHostFree(seen);
+    if (probed) (void)hipEventDestroy(probed);
   }
   void forget_seen() {
     if (seen) seen[0] = seen[1] = seen[2] = 0;
@@ -653,6 +654,9 @@ struct tmpm_session {
   }
   bool lists_paused = false;  // too many strays: full binnings for list_rest more reorder intervals
   uint32_t list_rest = 0, list_backoff = 1;
+  bool lists_probe = false;  // after a pause: few listed substeps per interval until their strays are known
+  bool probe_ran = false;    // all of an interval's are submitted, and `probed` follows them (if there is one)
+  hipEvent_t probed = nullptr;
   Topo topo{};
   uint32_t p2g_blocks = 4096, threads_pblock = 64, p2g_threads = 64;
   bool p2g_shape_fixed = false;  // P2G shape set by the tuner or an override, not by scene size
@@ -1767,7 +1771,7 @@ tmpm_status prepare_packed(tmpm_session* s, PackedParticles& pk) {
   st = alloc_topology(s, (uint32_t)pcap, (uint32_t)gcap);
   if (st != TMPM_OK) return st;
   s->substeps_since_reorder = 1u << 30;
-  s->lists_paused = false;
+  s->lists_paused = s->lists_probe = false;
   s->list_backoff = 1;
   s->compacted_last = false;
   s->prepared = true;
@@ -2033,21 +2037,30 @@ constexpr uint32_t kListSpan = 32;
 // that cross block faces as a whole stray all at once, and rarely.  Beyond it
 // substeps bin fully for a reorder interval, and for twice as many each time
 // that the lists are tried again and are no better.  The count is the device's:
-// substeps that are under way when the host first sees it are not changed.
+// substeps that are under way when the host first sees it are not changed.  A
+// trial is therefore kListProbe substeps of each interval until their count is
+// known.  A dense body in flight also strays, where more than kListRoom particles
+// a substep come into a block: 300,000 particles, 8 a cell, at 0.35 cells 320 / 180,
+// 1M, 16 a cell, 1,540 / 410.
 constexpr uint32_t kStraysMost = 600;  // a substep
 constexpr uint32_t kListRestMost = 64;
+constexpr uint32_t kListProbe = 2;
+
 void watch_strays(tmpm_session* s, bool synchronized) {
   if (!s->seen || s->lists_paused) return;
   const uint32_t span = std::min(s->reorder_interval, kListSpan) - 1;
-  if (((const volatile uint32_t*)s->seen)[2] <= kStraysMost * span) {
-    if (synchronized && s->lists_valid) s->list_backoff = 1;
-    return;
+  const uint32_t listed = s->lists_probe ? std::min(span, kListProbe) : span;
+  if (((const volatile uint32_t*)s->seen)[2] > kStraysMost * listed) {
+    s->seen[2] = 0;
+    s->lists_valid = s->lists_probe = false;
+    s->lists_paused = true;
+    s->list_rest = s->list_backoff;
+    s->list_backoff = std::min(2 * s->list_backoff, kListRestMost);
+  } else if (synchronized && s->lists_probe) {
+    s->lists_probe = !s->probe_ran;
+  } else if (synchronized && s->lists_valid) {
+    s->list_backoff = 1;
   }
-  s->seen[2] = 0;
-  s->lists_valid = false;
-  s->lists_paused = true;
-  s->list_rest = s->list_backoff;
-  s->list_backoff = std::min(2 * s->list_backoff, kListRestMost);
 }
 // The most obstacles or bodies for k_rigid_step's one workgroup: with 3 obstacles
 // 4.4 us against 9.6 of the three kernels it replaces (and two launches less),
@@ -2059,12 +2072,18 @@ SubstepPlan plan_substep(tmpm_session* s, bool apply_force, bool first, bool mor
   std::memset(&pl, 0, sizeof pl);
   pl.p = s->parts(s->cur);
   const bool scheduled = s->substeps_since_reorder >= s->reorder_interval;
-  watch_strays(s, false);
+  bool probed = false;  // the probe's substeps are done: their count is what the pinned words say
+  if (scheduled && s->lists_probe && s->probe_ran && s->probed) {
+    probed = hipEventQuery(s->probed) == hipSuccess;
+    if (!probed) (void)hipGetLastError();  // not ready is no error
+  }
+  watch_strays(s, probed);
   if (scheduled && s->lists_paused) {
     if (s->list_rest > 0) {
       --s->list_rest;
     } else {
-      s->lists_paused = false;
+      s->lists_paused = s->probe_ran = false;
+      s->lists_probe = true;
       if (s->seen) s->seen[2] = 0;  // a count from before the pause
     }
   }
@@ -2072,12 +2091,13 @@ SubstepPlan plan_substep(tmpm_session* s, bool apply_force, bool first, bool mor
   if (s->compacted_last) s->lists_last = !s->lists_dropped;  // the last substep reordered
   const bool use = more || s->lists_last;
   pl.reorder = scheduled ||
-               (may_list && !s->lists_valid && use && s->reorder_interval > 1 && s->reorder_interval <= kListSpan);
+               (may_list && !s->lists_probe && !s->lists_valid && use && s->reorder_interval > 1 && s->reorder_interval <= kListSpan);
   if (pl.reorder) pl.q = s->parts(1 - s->cur);
   pl.t = s->topo;
   const bool listed = !pl.reorder && may_list && s->lists_valid;
   const uint32_t since = pl.reorder ? 1u : s->substeps_since_reorder + 1;  // after this substep
-  const bool build = may_list && ((pl.reorder && use) || listed) && since < s->reorder_interval && since < kListSpan;
+  const bool build = may_list && ((pl.reorder && use) || listed) && since < s->reorder_interval &&
+                     since < (s->lists_probe ? kListProbe + 1 : kListSpan);
   pl.t.listed = listed ? 1 : 0;
   pl.t.build = build ? 1 : 0;
   const int read = listed ? s->list_read : 0;
@@ -2245,6 +2265,10 @@ hipError_t enqueue_substep(tmpm_session* s, bool apply_force, bool first, bool m
   if (e != hipSuccess) return e;
   s->lists_valid = pl.t.build != 0;
   s->lists_dropped = false;
+  if (s->lists_probe && pl.t.listed && !pl.t.build) {  // the last one of the probe
+    if (!s->probed && hipEventCreateWithFlags(&s->probed, hipEventDisableTiming) != hipSuccess) s->probed = nullptr;
+    s->probe_ran = !s->probed || hipEventRecord(s->probed, s->stream) == hipSuccess;
+  }
   s->rigid_pending = pl.rigid_next && !pl.rigid_step;
   s->list_read = pl.t.listed ? 1 - s->list_read : 1;
   s->table_dirty = pl.t.build != 0;  // otherwise G2P cleared the block table

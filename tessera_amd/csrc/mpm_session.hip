@@ -1108,6 +1108,7 @@ BlockLists block_lists(const tmpm_session* s, int set) {
 }
 
 constexpr uint32_t kRoomForSmall = 16384;  // blocks
+constexpr uint32_t kStraysMost = 600;      // a listed substep (watch_strays)
 
 // Allocates the topology for `pblocks` particle blocks and `gblocks` grid
 // blocks of capacity.
@@ -1686,6 +1687,25 @@ tmpm_status upload_classes(tmpm_session* s) {
 // enabled particles in insertion order, batches with room to admit more.
 tmpm_status prepare_packed(tmpm_session* s, PackedParticles& pk);
 
+// Strays a substep (watch_strays) that the uploaded state makes likely, from at
+// most 4,096 particles: those that change block, c on average per particle, and
+// beyond kListRoom of them into a block, or where blocks hold about one particle
+// each, so that a third of them find none where they go.  30,000 such particles
+// at 0.3 cells a substep had 1,100 (1,280 by this), 100,000 at 0.1 1,340 (1,420).
+double expected_strays(const tmpm_session* s, const PackedParticles& pk, uint64_t pblocks) {
+  const size_t n = pk.size(), step = n / 4096 + 1;
+  if (pblocks == 0) return 0.0;
+  double crossings = 0.0;
+  size_t seen = 0;
+  for (size_t i = 0; i < n; i += step, ++seen) {
+    const float4 v = pk.vv[i];
+    crossings += ((double)std::fabs(v.x) + std::fabs(v.y) + std::fabs(v.z)) * pk.inv_h[i] *
+                 s->scenes[pk.region[i] >> 16].substep_dt / kBlockCells;
+  }
+  const double c = crossings / seen, per_block = (double)n / pblocks;
+  return pblocks * std::max(c * per_block - (double)kListRoom, 0.0) + (per_block < 2.0 ? 0.35 * c * n : 0.0);
+}
+
 // Uploads every stepping scene.  A batch keeps the staging memory for later
 // admissions; a plain session frees it.
 tmpm_status prepare(tmpm_session* s) {
@@ -1771,7 +1791,8 @@ tmpm_status prepare_packed(tmpm_session* s, PackedParticles& pk) {
   st = alloc_topology(s, (uint32_t)pcap, (uint32_t)gcap);
   if (st != TMPM_OK) return st;
   s->substeps_since_reorder = 1u << 30;
-  s->lists_paused = s->lists_probe = false;
+  s->lists_paused = s->probe_ran = false;
+  s->lists_probe = expected_strays(s, pk, pblocks) > kStraysMost;
   s->list_backoff = 1;
   s->compacted_last = false;
   s->prepared = true;
@@ -2039,10 +2060,11 @@ constexpr uint32_t kListSpan = 32;
 // that the lists are tried again and are no better.  The count is the device's:
 // substeps that are under way when the host first sees it are not changed.  A
 // trial is therefore kListProbe substeps of each interval until their count is
-// known.  A dense body in flight also strays, where more than kListRoom particles
+// known, and so is the start of a session whose velocities make many likely
+// (expected_strays: by the mean block, so 16 a cell below, 508 -> 222 us in the
+// first submission of 32 substeps, not 8).  A dense body in flight also strays, where more than kListRoom particles
 // a substep come into a block: 300,000 particles, 8 a cell, at 0.35 cells 320 / 180,
 // 1M, 16 a cell, 1,540 / 410.
-constexpr uint32_t kStraysMost = 600;  // a substep
 constexpr uint32_t kListRestMost = 64;
 constexpr uint32_t kListProbe = 2;
 

@@ -2061,10 +2061,10 @@ constexpr uint32_t kListSpan = 32;
 // substeps that are under way when the host first sees it are not changed.  A
 // trial is therefore kListProbe substeps of each interval until their count is
 // known, and so is the start of a session whose velocities make many likely
-// (expected_strays: by the mean block, so 16 a cell below, 508 -> 222 us in the
-// first submission of 32 substeps, not 8).  A dense body in flight also strays, where more than kListRoom particles
-// a substep come into a block: 300,000 particles, 8 a cell, at 0.35 cells 320 / 180,
-// 1M, 16 a cell, 1,540 / 410.
+// (expected_strays).  A dense body in flight also strays, where more than
+// kListRoom particles a substep come into a block: 300,000 particles, 8 a cell, at
+// 0.35 cells a substep 320 / 180, 16 a cell 505 / 190 (508 and 222 in the first
+// submission of 32 substeps without and with a trial), 1M, 16 a cell, 1,540 / 410.
 constexpr uint32_t kListRestMost = 64;
 constexpr uint32_t kListProbe = 2;
 
